@@ -2937,7 +2937,12 @@ static int run_stages(int stages, const lia_attention_config *c, uint32_t n_seqs
         const uint32_t xcd = 1;
         const uint32_t cost = NT == kWideNT ? kUnitCostWide : kUnitCostDecode;
         const uint32_t lag = NT == kWideNT ? kLagWide : kLagDecode;
-        if (pk && n_seqs <= kPlanSeqs && n_wg <= kPlanThreads) {
+        // The parallel plan takes any number of workgroups (its descriptor loops stride); only its
+        // weighted range starts are an LDS table of kPlanThreads.  head_dim 64 decode launches 1,536
+        // workgroups (2,048 on FP8 pools): with the serial plan_kernel behind the two packing
+        // launches a step of 4 short sequences over two layers took 30.7 us, this way 22.6.
+        const bool parallel = n_seqs <= kPlanSeqs && (!lag || n_wg <= kPlanThreads);
+        if (pk && parallel) {
             // the packing, the plan (from the packing's inputs) and the table checks in one
             // launch, then the step's verdict
             const RawSeqs raw{pk->q_lens, pk->cached, pk->seq_slots, n_rows};
@@ -2949,19 +2954,17 @@ static int run_stages(int stages, const lia_attention_config *c, uint32_t n_seqs
                                                  pk->cu, pk->slot_mapping, pk->status, header, work, n_wg,
                                                  merge, L.max_units);
         } else {
-            if (pk) { // too many sequences or workgroups for the one-launch form: pack first
+            if (pk) { // too many sequences for the one-launch form: pack first
                 const int ps = lia_pack_device(n_seqs, pk->seq_slots, pk->q_lens, pk->cached, pk->pages,
                                                pk->stride, 1u << pk->page_shift, pk->pool_pages,
                                                pk->context, pk->max_rows, pk->cu, pk->positions,
                                                pk->sequences, pk->slot_mapping, pk->status, stream);
                 if (ps) return ps;
             }
-            if (n_seqs <= kPlanSeqs && n_wg <= kPlanThreads)
+            if (parallel)
             e = launch<plan_lds_kernel>(dim3(kPlanGroups), dim3(kPlanThreads), 0, s, n_seqs, cu_seqlens,
                                         positions, sequences, pages, c->stride, p.page_shift, rpc,
-                                        c->num_kv_heads, L.max_units, n_wg,
-                                        NT == kWideNT ? kUnitCostWide : kUnitCostDecode,
-                                        lia_device_cus(), NT == kWideNT ? kLagWide : kLagDecode,
+                                        c->num_kv_heads, L.max_units, n_wg, cost, lia_device_cus(), lag,
                                         xcd, units, work, merge, header);
             else
             e = launch<plan_kernel>(dim3(1), dim3(256), 0, s, n_seqs, cu_seqlens, positions,

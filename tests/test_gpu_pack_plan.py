@@ -144,3 +144,24 @@ def test_pack_plan_rows_over_capacity_and_row_count_mismatch(lia, wl):
         assert int(status.item()) == want
         # nothing planned: an over-capacity batch (rejected) and a row count other than n_rows
         assert hdr[0] == 0 and hdr[2] == 0, (q, hdr)
+
+
+@pytest.mark.parametrize("n", [1, 5, 64, 300])
+def test_pack_plan_head_dim_64_decode(lia, wl, n):
+    """head_dim 64 decode launches more workgroups (1,536) than the plan has threads (1,024): the
+    one-launch form equals pack-then-plan bit for bit and the float64 oracle to the bf16 bar, with
+    fewer blocks than workgroups, about as many, and several per workgroup."""
+    rng = np.random.default_rng(64 + n)
+    ctx = np.exp(rng.uniform(np.log(2), np.log(1500 if n > 5 else 9000), n)).astype(np.int64)
+    b = wl.custom(ctx, [1] * n, geom=wl.Geometry(hq=8, hkv=2, d=64), seed=64 + n)
+    case = G.Case(b, seed=64 + n)
+    cfg = case.config(lia)
+    print(f"[case] pack+plan head_dim 64: seqs={n} keys={int(ctx.sum())}", flush=True)
+    ref = _run(lia, b, case, False, b.flat_table(), cfg, fused_append=False)
+    got = _run(lia, b, case, True, b.flat_table(), cfg, fill_ws=0xA5, fused_append=False)
+    for key in ("status", "cu", "positions", "sequences", "slots", "out"):
+        assert np.array_equal(got[key], ref[key]), key
+    assert np.array_equal(got["header"][:5], ref["header"][:5]) and got["header"][3] == 0
+    out = torch.from_numpy(got["out"]).view(torch.bfloat16).float().numpy()
+    mx, mean = G.errors(out, case.f64())
+    assert mx < 2e-2 and mean < 2e-3, (mx, mean)
