@@ -122,43 +122,34 @@ __device__ __forceinline__ uint32_t unit_blocks(uint32_t p0, uint32_t new_keys) 
     return (p0 + 31) / 32 + (new_keys + 31) / 32;
 }
 
-// sum_{i=0}^{n-1} floor((a*i + b) / m) (the standard floor-sum reduction, O(log) steps),
-// for the plan's small operands: 32-bit divisions, 64-bit sum.
-__device__ __forceinline__ uint64_t floor_sum(uint32_t n, uint32_t m, uint32_t a, uint32_t b) {
-    uint64_t ans = 0;
-    while (true) {
-        if (a >= m) {
-            ans += (uint64_t)n * (n - 1) / 2 * (a / m);
-            a %= m;
-        }
-        if (b >= m) {
-            ans += (uint64_t)n * (b / m);
-            b %= m;
-        }
-        const uint32_t y = a * n + b;
-        if (y < m) break;
-        n = y / m;
-        b = y % m;
-        const uint32_t tmp = m;
-        m = a;
-        a = tmp;
-    }
-    return ans;
-}
-
 // New-key blocks of column blocks 0 .. m-1 of a sequence in one KV head: sum over c = 1..m
 // of ceil(c * rpc / 32) (column block c-1 ends at row c * rpc, before the last block).
-// Power-of-two rpc (every batch shape the launches choose) in closed form with k = 32/rpc:
-// k*q*(q+1)/2 + r*(q+1), q = m / k, r = m % k.
+// Power-of-two rpc (every group that is one) in closed form with k = 32/rpc:
+// k*q*(q+1)/2 + r*(q+1), q = m / k, r = m % k.  Otherwise the sum is (rpc * m(m+1)/2 + R(m)) / 32
+// with R(m) the sum of the residues (-c * rpc) mod 32: over a period of k = 32/gcd(rpc, 32) they
+// are the multiples of 32/k once each, 16(k-1) in all, and the rest (below 32 terms) is summed.
 __device__ __forceinline__ uint32_t new_blocks_before(uint32_t m, uint32_t rpc) {
-    if (!m) return 0;
-    if ((rpc & (rpc - 1)) == 0) {
+    const uint32_t low = rpc & (0u - rpc); // the largest power of two in rpc
+    if (low == rpc) {
         if (rpc >= 32) return (rpc >> 5) * (m * (m + 1) / 2);
         const uint32_t lk = 5 - (31 - __builtin_clz(rpc)), k = 1u << lk; // k = 32 / rpc
         const uint32_t q = m >> lk, r = m & (k - 1);
         return k * q * (q + 1) / 2 + r * (q + 1);
     }
-    return (uint32_t)floor_sum(m, 32, rpc, rpc + 31);
+    const uint32_t lk = low >= 32 ? 0u : 5 - (31 - __builtin_clz(low)), k = 1u << lk;
+    uint32_t res = (m >> lk) * 16 * (k - 1);
+#pragma unroll 1
+    for (uint32_t c = m & (k - 1); c; c--) res += (0u - c * rpc) & 31u;
+    return (uint32_t)(((uint64_t)rpc * m * (m + 1) / 2 + res) >> 5);
+}
+
+// floor(a / b) for a < 2^53 and quotients below 2^32, with inv = 1.0 / b: the product is off by
+// less than one, which the remainder settles (a 64-bit division is a long software sequence, and
+// the plan is one pass over cold code).
+__device__ __forceinline__ uint32_t div_by(uint64_t a, uint64_t b, double inv) {
+    const uint32_t q = (uint32_t)((double)a * inv);
+    const int64_t rem = (int64_t)(a - q * b);
+    return rem < 0 ? q - 1 : (uint64_t)rem >= b ? q + 1 : q;
 }
 
 constexpr uint32_t kPlanSeqs = 1024; // sequences the plan keeps in LDS (one per thread)
@@ -204,21 +195,26 @@ struct RawSeqs {
     uint32_t n_rows;
 };
 
-__device__ void plan_lds(uint32_t n_seqs, const uint32_t *cu, const uint32_t *positions,
-                         const uint32_t *sequences, const RawSeqs *raw, const uint32_t *pages,
-                         uint32_t stride, uint32_t page_shift, uint32_t rpc, uint32_t hkv,
-                         uint32_t max_units, uint32_t n_wg, uint32_t unit_cost, uint32_t round_wg,
-                         uint32_t lag, uint32_t xcd, uint32_t grp, uint32_t ngrp, UnitDesc *units,
-                         WorkDesc *work, MergeDesc *merge, uint32_t *header) {
+template <bool RAW>
+__device__ __forceinline__ void plan_lds(uint32_t n_seqs, const uint32_t *cu, const uint32_t *positions,
+                                         const uint32_t *sequences, const RawSeqs &raw,
+                                         const uint32_t *pages, uint32_t stride, uint32_t page_shift,
+                                         uint32_t rpc, uint32_t hkv, uint32_t max_units, uint32_t n_wg,
+                                         uint32_t unit_cost, uint32_t round_wg, uint32_t lag, uint32_t xcd,
+                                         uint32_t grp, uint32_t ngrp, UnitDesc *units, WorkDesc *work,
+                                         MergeDesc *merge, uint32_t *header) {
+    // per sequence: first packed row, rows, cached keys, table row, column blocks, blocks of one KV
+    // head; and the running sums of its units, blocks and cost
     __shared__ uint32_t s_r0[kPlanSeqs], s_nr[kPlanSeqs], s_p0[kPlanSeqs], s_trow[kPlanSeqs];
+    __shared__ uint32_t s_ncb[kPlanSeqs], s_nbh[kPlanSeqs];
     __shared__ uint32_t s_u0[kPlanSeqs + 1], s_b0[kPlanSeqs + 1], s_c0[kPlanSeqs + 1];
     __shared__ uint32_t w_s[4][kPlanThreads / 64];
     __shared__ uint32_t carry_units, carry_blocks, carry_rows, raw_bad;
-    __shared__ uint64_t s_rlo[kPlanThreads + 1];
+    __shared__ uint32_t s_rlo[kPlanThreads + 1];
     // Threads exchange only LDS data (nothing written to global memory is read back), so the
     // barriers need not wait for the descriptor stores in flight.
     constexpr uint32_t T = kPlanThreads;
-    const uint32_t t = threadIdx.x;
+    const uint32_t t = threadIdx.x, lane = t & 63;
     // the workgroups of the launch share the descriptor loops; each computes the per-sequence
     // extents and range starts itself (they live in its LDS)
     const uint32_t g0 = t * ngrp + grp, GT = ngrp * T; // interleaved shares
@@ -227,14 +223,14 @@ __device__ void plan_lds(uint32_t n_seqs, const uint32_t *cu, const uint32_t *po
     const uint32_t last = one_wave ? 63 : T - 1; // the thread holding the totals
     {
         const uint32_t b = t;
-        uint32_t nu = 0, nb = 0, r0 = 0, nr = 0, p0 = 0, trow = 0;
+        uint32_t nu = 0, nb = 0, r0 = 0, nr = 0, p0 = 0, trow = 0, ncb = 0, nbh = 0;
         if (b < n_seqs) {
-            if (raw) {
+            if constexpr (RAW) {
                 // the packing's inputs; the rows before this sequence are a scan of the
                 // new-token counts, below
-                nr = raw->q_lens[b];
-                p0 = raw->cached[b];
-                trow = raw->seq_slots[b];
+                nr = raw.q_lens[b];
+                p0 = raw.cached[b];
+                trow = raw.seq_slots[b];
             } else {
                 r0 = cu[b];
                 nr = cu[b + 1] - r0;
@@ -244,9 +240,10 @@ __device__ void plan_lds(uint32_t n_seqs, const uint32_t *cu, const uint32_t *po
                 }
             }
             if (nr > 0) {
-                const uint32_t ncb = (nr + rpc - 1) / rpc;
+                ncb = (nr + rpc - 1) / rpc;
+                nbh = ncb * ((p0 + 31) / 32) + new_blocks_before(ncb - 1, rpc) + (nr + 31) / 32;
                 nu = ncb * hkv;
-                nb = (ncb * ((p0 + 31) / 32) + new_blocks_before(ncb - 1, rpc) + (nr + 31) / 32) * hkv;
+                nb = nbh * hkv;
             }
         }
         // inclusive scans of the units and blocks, and on raw inputs of the rows and of the
@@ -254,23 +251,25 @@ __device__ void plan_lds(uint32_t n_seqs, const uint32_t *cu, const uint32_t *po
         // validated its inputs: such a sequence makes the plan empty, so no table read leaves
         // the row.
         uint32_t v[4] = {nu, nb, nr,
-                         raw && (uint64_t)p0 + nr > ((uint64_t)stride << page_shift) ? 1u : 0u};
-        if (raw) block_scan_n<4>(v, w_s, one_wave);
-        else block_scan_n<2>(v, w_s, one_wave);
-        if (raw) r0 = v[2] - nr;
+                         RAW && (uint64_t)p0 + nr > ((uint64_t)stride << page_shift) ? 1u : 0u};
+        block_scan_n<RAW ? 4 : 2>(v, w_s, one_wave);
+        if constexpr (RAW) r0 = v[2] - nr;
         if (b < n_seqs) {
             s_r0[b] = r0; s_nr[b] = nr; s_p0[b] = p0; s_trow[b] = trow;
+            s_ncb[b] = ncb;
+            s_nbh[b] = nbh;
             s_u0[b] = v[0] - nu;
             s_b0[b] = v[1] - nb;
             s_c0[b] = v[1] - nb + unit_cost * (v[0] - nu);
         }
         if (t == last) {
             carry_units = v[0]; carry_blocks = v[1];
-            if (raw) { carry_rows = v[2]; raw_bad = v[3]; }
+            if constexpr (RAW) { carry_rows = v[2]; raw_bad = v[3]; }
         }
         lds_barrier();
     }
-    const bool overflow = carry_units > max_units || (raw && (carry_rows != raw->n_rows || raw_bad));
+    bool overflow = carry_units > max_units;
+    if constexpr (RAW) overflow |= carry_rows != raw.n_rows || raw_bad;
     const uint32_t U = overflow ? 0 : carry_units, B = overflow ? 0 : carry_blocks;
     const uint32_t N = min(n_wg, B);
     if (t == 0) {
@@ -285,33 +284,9 @@ __device__ void plan_lds(uint32_t n_seqs, const uint32_t *cu, const uint32_t *po
             header[3] = overflow;
             // the batch verdict: a plan of packed metadata is never of a rejected batch (its
             // rejection empties cu_seqlens); the packing beside a raw plan writes it instead
-            if (!raw) header[kVerdict] = 0;
+            if constexpr (!RAW) header[kVerdict] = 0;
         }
     }
-    lds_barrier();
-    // last sequence b with arr[b] <= v (empty sequences share their offset with the next
-    // one, so this is the sequence that owns v)
-    auto seq_of = [&](const uint32_t *arr, uint32_t v) {
-        uint32_t a = 0, e = n_seqs;
-        while (a + 1 < e) {
-            const uint32_t mid = (a + e) >> 1;
-            if (arr[mid] <= v) a = mid; else e = mid;
-        }
-        return a;
-    };
-    auto make_unit = [&](uint32_t b, uint32_t h, uint32_t cb) {
-        const uint32_t nr = s_nr[b], p0 = s_p0[b], cblocks = (p0 + 31) / 32;
-        const uint32_t nbh = (s_b0[b + 1] - s_b0[b]) / hkv;
-        const uint32_t rows = min(rpc, nr - cb * rpc), kend = p0 + cb * rpc + rows;
-        const uint32_t blk = s_b0[b] + h * nbh + cb * cblocks + new_blocks_before(cb, rpc);
-        return UnitDesc{blk, unit_blocks(p0, kend - p0), cblocks, s_r0[b] + cb * rpc, rows | (h << 16),
-                        kend, s_trow[b], p0};
-    };
-    auto unit_by_index = [&](uint32_t u) {
-        const uint32_t b = seq_of(s_u0, u), ncb = (s_nr[b] + rpc - 1) / rpc, i = u - s_u0[b];
-        return make_unit(b, i / ncb, i % ncb);
-    };
-    const uint32_t P = 1u << page_shift;
     for (uint32_t w = N + g0; w < n_wg; w += GT) { // launched workgroups without work
         WorkDesc d = {};
         work[w] = d;
@@ -329,124 +304,129 @@ __device__ void plan_lds(uint32_t n_seqs, const uint32_t *cu, const uint32_t *po
     // hardware issues first, so its range is weighted (256 - lag) / 256 against 1 for the first
     // round (lag 0: equal shares).  F(r) = sum of the weights of ranges before r, times 256.
     auto late_before = [&](uint32_t r) -> uint32_t { // ranges before r on workgroups w >= round_wg
-        uint32_t late = 0;
-        if (xcd_major) {
-            const uint32_t X = r / per, I = r % per;
-            for (uint32_t x = 0; x <= X && x < 8; x++) {
-                const uint32_t cx = round_wg > x ? min(per, (round_wg - x + 7) / 8) : 0u;
-                late += x < X ? per - cx : (I > cx ? I - cx : 0u);
-            }
-        } else {
-            late = r > round_wg ? r - round_wg : 0u;
-        }
-        return late;
+        if (!xcd_major) return r > round_wg ? r - round_wg : 0u;
+        // XCD x runs ranges x * per + i on workgroups 8i + x: the first ceil((round_wg - x) / 8)
+        const uint32_t X = r / per, I = r % per, early = round_wg / 8, more = round_wg % 8;
+        const uint32_t a = min(per, early + 1), b = min(per, early);
+        return min(X, more) * (per - a) + (X - min(X, more)) * (per - b) +
+               (I > (X < more ? a : b) ? I - (X < more ? a : b) : 0u);
     };
     // Weights only when every range still spans at least one block of cost: a range weighted w
     // of 256 spans TC * w / F(N) >= TC * (256 - lag) / F(N), so with that at least 1 each start
     // lies at least one block after the previous one.  A range empty in blocks inside a unit
     // would be counted among the unit's records without writing one.
-    const bool skew = lag && round_wg && round_wg < N &&
-                      TC * (256 - lag) >= 256ull * N - (uint64_t)lag * late_before(N);
-    auto weight_before = [&](uint32_t r) -> uint64_t {
-        return 256ull * r - (skew ? (uint64_t)lag * late_before(r) : 0ull);
-    };
-    // Equal weights: range r starts at cost r*TC/N, and cost c lies in range ((c+1)*N-1)/TC.
-    // Weighted: the start cost of every range is tabulated once (one division per range) and
-    // searched.
+    bool skew = lag && round_wg && round_wg < N;
+    uint64_t FN = N; // the weights' sum (equal weights: one each)
     if (skew) {
-        const uint64_t FN = weight_before(N);
-        for (uint32_t r = t; r <= N; r += T) s_rlo[r] = weight_before(r) * TC / FN;
-        lds_barrier();
+        const uint64_t weighted = 256ull * N - (uint64_t)lag * late_before(N);
+        skew = TC * (256 - lag) >= weighted;
+        if (skew) FN = weighted;
     }
-    // equal shares in 32-bit arithmetic when TC * N fits (every batch up to 2^32 / n_wg
-    // blocks): a 64-bit division is a long software sequence on the plan's critical path
-    const bool narrow = TC * N < (1ull << 32);
-    auto range_lo = [&](uint32_t r) -> uint64_t {
-        if (skew) return s_rlo[r];
-        return narrow ? r * (uint32_t)TC / N : (uint64_t)r * TC / N;
-    };
-    // the last range starting at or before cost c
-    auto range_of = [&](uint64_t c) {
-        if (!skew) return narrow ? ((uint32_t)c * N + N - 1) / (uint32_t)TC : (uint32_t)(((c + 1) * N - 1) / TC);
-        uint32_t a = 0, e = N;
+    // Equal weights: range r starts at cost r*TC/N, and cost c lies in range ((c+1)*N-1)/TC.
+    // Weighted: the start cost of every range is tabulated once and searched.
+    const double inv_n = 1.0 / (double)FN, inv_tc = 1.0 / (double)TC;
+    if (skew) {
+        for (uint32_t r = t; r <= N; r += T)
+            s_rlo[r] = div_by((256ull * r - (uint64_t)lag * late_before(r)) * TC, FN, inv_n);
+    }
+    lds_barrier();
+    auto range_lo = [&](uint32_t r) -> uint32_t { return skew ? s_rlo[r] : div_by(r * TC, FN, inv_n); };
+    // last index a of arr[0 .. n) (ascending, arr[0] <= v) with arr[a] <= v.  On sequences: empty
+    // ones share their offset with the next, so this is the sequence that owns v.
+    auto last_le = [&](const uint32_t *arr, uint32_t n, uint32_t v) {
+        uint32_t a = 0, e = n;
+#pragma unroll 1
         while (a + 1 < e) {
             const uint32_t mid = (a + e) >> 1;
-            if (s_rlo[mid] <= c) a = mid; else e = mid;
+            if (arr[mid] <= v) a = mid; else e = mid;
         }
         return a;
     };
+    auto make_unit = [&](uint32_t b, uint32_t h, uint32_t cb) {
+        const uint32_t p0 = s_p0[b], cblocks = (p0 + 31) / 32;
+        const uint32_t rows = min(rpc, s_nr[b] - cb * rpc), kend = p0 + cb * rpc + rows;
+        const uint32_t blk = s_b0[b] + h * s_nbh[b] + cb * cblocks + new_blocks_before(cb, rpc);
+        return UnitDesc{blk, unit_blocks(p0, kend - p0), cblocks, s_r0[b] + cb * rpc, rows | (h << 16),
+                        kend, s_trow[b], p0};
+    };
+    // The work descriptors, 63 ranges to a wave (each lane finds its range's start, and takes the
+    // next range's from the next lane), by the last waves, so that their chain (searches, table
+    // loads) runs beside the units' on the others.  Each workgroup takes contiguous ranges.
+    const uint32_t share = (N + ngrp - 1) / ngrp, wave = (T - 1 - t) >> 6;
+#pragma unroll 1
+    for (uint32_t r0 = wave * 63; r0 < share; r0 += 63 * (T / 64)) {
+        const uint32_t r = grp * share + r0 + lane;
+        const uint32_t c = r < N ? range_lo(r) : (uint32_t)TC;
+        // The block at cost c, and its unit (sequence b, KV head h, column block cb): in cost,
+        // sequence b starts at s_c0[b], a KV head's units span nbh + unit_cost * ncb, and a unit's
+        // blocks follow its unit_cost lead-in; a cost inside a lead-in maps to the unit's first block.
+        uint32_t b = 0, h = 0, cb = 0, lo = B;
+        if (r < N) {
+            b = last_le(s_c0, n_seqs, c);
+            const uint32_t ncb = s_ncb[b], cblocks = (s_p0[b] + 31) / 32, nbh = s_nbh[b];
+            const uint32_t hsp = nbh + unit_cost * ncb, co = c - s_c0[b];
+            h = co / hsp;
+            const uint32_t in = co - h * hsp;
+            uint32_t e = ncb; // last cb whose cost start is at or before it
+#pragma unroll 1
+            while (cb + 1 < e) {
+                const uint32_t mid = (cb + e) >> 1;
+                if (mid * cblocks + new_blocks_before(mid, rpc) + unit_cost * mid <= in) cb = mid; else e = mid;
+            }
+            const uint32_t ustart = cb * cblocks + new_blocks_before(cb, rpc);
+            const uint32_t off = in - (ustart + unit_cost * cb);
+            lo = s_b0[b] + h * nbh + ustart + (off < unit_cost ? 0u : off - unit_cost);
+        }
+        const uint32_t hi = __shfl_down(lo, 1);
+        if (lane == 63 || r >= N || r0 + lane >= share) continue;
+        WorkDesc d;
+        d.unit = s_u0[b] + h * s_ncb[b] + cb;
+        d.first = make_unit(b, h, cb);
+        d.flags = r << 8;
+        d.lo = lo;
+        d.hi = hi;
+        // logical pages the range starts with, when it starts in the cached keys (unconditional
+        // page-table loads: an entry not needed reads a word the plan reads anyway - cu[0], or
+        // q_lens[0] of a raw plan - and is replaced by 0)
+        const uint32_t *dummy = RAW ? raw.q_lens : cu;
+        const uint32_t rel = lo - d.first.block_start;
+        const bool pre = pages && rel < d.first.cblocks;
+        const uint32_t lp = (32 * rel) >> page_shift;
+        const uint32_t lend = (d.first.kend + (1u << page_shift) - 1) >> page_shift;
+        uint32_t v[kPrePages];
+#pragma unroll
+        for (uint32_t i = 0; i < kPrePages; i++) {
+            const bool use = pre && lp + i < lend;
+            const uint32_t *src = use ? pages + (size_t)d.first.table_row * stride + lp + i : dummy;
+            v[i] = *src;
+            v[i] = use ? v[i] : 0u;
+        }
+        if (pre) d.flags |= 1;
+        d.pre = make_uint4(v[0], v[1], v[2], v[3]);
+        work[xcd_major ? (r % per) * 8 + r / per : r] = d;
+    }
     // each unit's descriptor, and its merge descriptor from it
+#pragma unroll 1
     for (uint32_t u = g0; u < max_units; u += GT) {
         MergeDesc m = {0, 0, 0, 0};
         if (u < U) {
-            const UnitDesc ud = unit_by_index(u);
+            const uint32_t b = last_le(s_u0, n_seqs, u), ncb = s_ncb[b], i = u - s_u0[b];
+            const uint32_t h = i / ncb;
+            const UnitDesc ud = make_unit(b, h, i - h * ncb);
             units[u] = ud;
-            const uint64_t cu0 = (uint64_t)ud.block_start + unit_cost * (u + 1); // cost of its first block
-            const uint32_t wf = range_of(cu0), wl = range_of(cu0 + ud.nblocks - 1);
+            // the ranges of its first and last block: the last ranges starting at or before them
+            const uint32_t cf = ud.block_start + unit_cost * (u + 1), cl = cf + ud.nblocks - 1;
+            uint32_t wf, wl;
+            if (skew) {
+                wf = last_le(s_rlo, N, cf);
+                wl = last_le(s_rlo, N, cl);
+            } else {
+                wf = div_by((uint64_t)(cf + 1) * N - 1, TC, inv_tc);
+                wl = div_by((uint64_t)(cl + 1) * N - 1, TC, inv_tc);
+            }
             if (wf != wl) m = MergeDesc{wf + u, wl - wf + 1, ud.rowbeg, ud.nrows_hk};
         }
         merge[u] = m;
-    }
-    // The block at cost c, and its unit (sequence ub, KV head uh, column block ucb): in cost,
-    // sequence b starts at s_c0[b], a KV head's units span nbh + unit_cost * ncb, and a unit's
-    // blocks follow its unit_cost lead-in; a cost inside a lead-in maps to the unit's first block.
-    auto block_of_cost = [&](uint64_t c, uint32_t &ub, uint32_t &uh, uint32_t &ucb) {
-        if (c >= TC) { ub = n_seqs; return B; }
-        const uint32_t cc = (uint32_t)c;
-        const uint32_t b = seq_of(s_c0, cc);
-        const uint32_t ncb = (s_nr[b] + rpc - 1) / rpc, cblocks = (s_p0[b] + 31) / 32;
-        const uint32_t nbh = (s_b0[b + 1] - s_b0[b]) / hkv;
-        const uint32_t hsp = nbh + unit_cost * ncb, co = cc - s_c0[b];
-        const uint32_t h = co / hsp, co2 = co - h * hsp;
-        uint32_t cb = 0, e = ncb; // last cb whose cost start <= co2
-        while (cb + 1 < e) {
-            const uint32_t mid = (cb + e) >> 1;
-            if (mid * cblocks + new_blocks_before(mid, rpc) + unit_cost * mid <= co2) cb = mid; else e = mid;
-        }
-        const uint32_t ustart = cb * cblocks + new_blocks_before(cb, rpc);
-        const uint32_t off = co2 - (ustart + unit_cost * cb);
-        ub = b; uh = h; ucb = cb;
-        return s_b0[b] + h * nbh + ustart + (off < unit_cost ? 0u : off - unit_cost);
-    };
-    // One work descriptor per thread and pass (unconditional page-table loads: an entry not
-    // needed reads a word the plan reads anyway - cu[0], or q_lens[0] of a raw plan, whose
-    // cu is null - and is replaced by 0).
-    const uint32_t *dummy = raw ? raw->q_lens : cu;
-    // the work descriptors from the last threads, so that their chain (searches, divisions,
-    // table loads) runs beside the units' on other waves
-    for (uint32_t w0 = (T - 1 - t) * ngrp + grp; w0 < N; w0 += GT) {
-        WorkDesc d[1];
-        uint32_t v[1][kPrePages];
-        {
-            constexpr int k = 0;
-            const uint32_t w = w0;
-            const uint32_t r = xcd_major ? (w % 8) * per + w / 8 : w;
-            uint32_t b, h, c, b2, h2, c2;
-            const uint32_t lo = block_of_cost(range_lo(r), b, h, c);
-            const uint32_t hi = block_of_cost(range_lo(r + 1), b2, h2, c2);
-            if (b >= n_seqs) { b = 0; h = 0; c = 0; } // empty range at the end
-            const uint32_t ncb = (s_nr[b] + rpc - 1) / rpc;
-            d[k].unit = s_u0[b] + h * ncb + c;
-            d[k].first = make_unit(b, h, c);
-            d[k].flags = r << 8;
-            d[k].lo = lo;
-            d[k].hi = hi;
-            // logical pages the range starts with, when it starts in the cached keys
-            const uint32_t rel = lo - d[k].first.block_start;
-            const bool pre = pages && rel < d[k].first.cblocks;
-            const uint32_t lp = (32 * rel) >> page_shift;
-            const uint32_t lend = (d[k].first.kend + P - 1) >> page_shift;
-#pragma unroll
-            for (uint32_t i = 0; i < kPrePages; i++) {
-                const bool use = pre && lp + i < lend;
-                const uint32_t *src = use ? pages + (size_t)d[k].first.table_row * stride + lp + i : dummy;
-                v[k][i] = *src;
-                v[k][i] = use ? v[k][i] : 0u;
-            }
-            if (pre) d[k].flags |= 1;
-        }
-        d[0].pre = make_uint4(v[0][0], v[0][1], v[0][2], v[0][3]);
-        work[w0] = d[0];
     }
 }
 
@@ -455,7 +435,7 @@ __global__ __launch_bounds__(kPlanThreads) void plan_lds_kernel(
     const uint32_t *pages, uint32_t stride, uint32_t page_shift, uint32_t rpc, uint32_t hkv,
     uint32_t max_units, uint32_t n_wg, uint32_t unit_cost, uint32_t round_wg, uint32_t lag,
     uint32_t xcd, UnitDesc *units, WorkDesc *work, MergeDesc *merge, uint32_t *header) {
-    plan_lds(n_seqs, cu, positions, sequences, nullptr, pages, stride, page_shift, rpc, hkv, max_units,
+    plan_lds<false>(n_seqs, cu, positions, sequences, RawSeqs{}, pages, stride, page_shift, rpc, hkv, max_units,
              n_wg, unit_cost, round_wg, lag, xcd, blockIdx.x, gridDim.x, units, work, merge, header);
 }
 
@@ -479,7 +459,7 @@ __global__ __launch_bounds__(kPlanThreads) void pack_plan_kernel(
     WorkDesc *work, MergeDesc *merge, uint32_t *header) {
     const uint32_t bid = blockIdx.x;
     if (bid < kPlanGroups) {
-        plan_lds(n_seqs, nullptr, nullptr, nullptr, &raw, pk.pages, pk.stride, pk.page_shift, rpc, hkv,
+        plan_lds<true>(n_seqs, nullptr, nullptr, nullptr, raw, pk.pages, pk.stride, pk.page_shift, rpc, hkv,
                  max_units, n_wg, unit_cost, round_wg, lag, xcd, bid, kPlanGroups, units, work, merge,
                  header);
     } else if (bid == kPlanGroups) {
