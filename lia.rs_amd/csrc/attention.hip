@@ -183,13 +183,36 @@ constexpr uint32_t kLagWide = 56, kLagDecode = 0;
 // in LDS (a shuffle scan with one barrier) and every unit in closed form (unit (h, cb) of
 // sequence b starts at block b0 + h*nbh + cb*cblocks + new_blocks_before(cb)), so units, merge
 // descriptors and the work list are each written in parallel with no serial per-sequence loop
-// and no reads of the units just written.  Workgroups get shares of cost - the blocks plus
-// unit_cost per unit (its start) - equal, or weighted by dispatch round (round_wg, lag).
+// and no reads of the units just written.  Workgroups get ranges by the PlanRule.
 //
 // Per-sequence extents come from the packed metadata (cu_seqlens, positions, sequences), or,
 // with `raw` set, from the packing's own inputs (raw->q_lens, cached, seq_slots), so the plan
 // can run beside the packing in one launch; a raw batch whose rows differ from raw->n_rows is
 // planned empty.  The workgroup is `grp` of `ngrp` sharing the descriptor loops.
+
+// How a plan divides its cost (blocks plus unit_cost per unit) over workgroups.  Ranges of equal
+// cost over every resident workgroup, weighted by dispatch round (round_wg, lag), are best while
+// each range spans many blocks.  On small batches (cost below small_cost) two costs of a split
+// show instead: a range's start, and the records its units leave for the combine.
+//  - Decode: at least two blocks of cost to a range (one costs up to 15 %: three rows on 9,000
+//    keys, two layers, 36.9 -> 32.0 us; 32 rows on 100-800 FP8 keys 40.7 -> 36.9; three lose 1-2 us
+//    on contexts below 4,000 keys).
+//  - One range per unit, which leaves no records, when that costs less: the longest unit against
+//    an even share plus the records.  Decode: at most 4 blocks above the share, less on batches of
+//    few records (64 short rows of 8 KV heads 32.9 -> 28.3 us; few units are faster split).
+//    Prefill, in eighths of the time two workgroups sharing a CU take for a block of each (0.45
+//    us): a block of a workgroup alone on its CU costs 13 (0.71 us); above one unit per CU the
+//    even share of the blocks, and 12 % for uneven pairs, counts too; a record costs 4.5/16 in 16
+//    bits and 9/16 in f32 (written and read at 5 TB/s).  4 chunks of 512 rows, 32 query / 8 KV
+//    heads, from empty caches 52.6 -> 37.4 us, on 4,000 keys 181.8 -> 159.4; 8 of 256 rows on
+//    4,000 keys 201 -> 156; two heads and 256 units on 4,000 keys stay split (97 us; 122 unsplit).
+struct PlanRule {
+    uint32_t unit_cost;  // virtual blocks charged to each unit
+    uint32_t round_wg, lag, xcd;
+    uint32_t small_cost, span_shift;
+    uint32_t rec;        // prefill: a record's cost (16ths of an eighth of a block); decode: 0
+};
+
 struct RawSeqs {
     const uint32_t *q_lens, *cached, *seq_slots;
     uint32_t n_rows;
@@ -200,21 +223,20 @@ __device__ __forceinline__ void plan_lds(uint32_t n_seqs, const uint32_t *cu, co
                                          const uint32_t *sequences, const RawSeqs &raw,
                                          const uint32_t *pages, uint32_t stride, uint32_t page_shift,
                                          uint32_t rpc, uint32_t hkv, uint32_t max_units, uint32_t n_wg,
-                                         uint32_t unit_cost, uint32_t round_wg, uint32_t lag, uint32_t xcd,
-                                         uint32_t grp, uint32_t ngrp, UnitDesc *units, WorkDesc *work,
-                                         MergeDesc *merge, uint32_t *header) {
+                                         const PlanRule &rule, uint32_t grp, uint32_t ngrp, UnitDesc *units,
+                                         WorkDesc *work, MergeDesc *merge, uint32_t *header) {
     // per sequence: first packed row, rows, cached keys, table row, column blocks, blocks of one KV
     // head; and the running sums of its units, blocks and cost
     __shared__ uint32_t s_r0[kPlanSeqs], s_nr[kPlanSeqs], s_p0[kPlanSeqs], s_trow[kPlanSeqs];
     __shared__ uint32_t s_ncb[kPlanSeqs], s_nbh[kPlanSeqs];
     __shared__ uint32_t s_u0[kPlanSeqs + 1], s_b0[kPlanSeqs + 1], s_c0[kPlanSeqs + 1];
-    __shared__ uint32_t w_s[4][kPlanThreads / 64];
+    __shared__ uint32_t w_s[4][kPlanThreads / 64], w_long[kPlanThreads / 64];
     __shared__ uint32_t carry_units, carry_blocks, carry_rows, raw_bad;
     __shared__ uint32_t s_rlo[kPlanThreads + 1];
     // Threads exchange only LDS data (nothing written to global memory is read back), so the
     // barriers need not wait for the descriptor stores in flight.
     constexpr uint32_t T = kPlanThreads;
-    const uint32_t t = threadIdx.x, lane = t & 63;
+    const uint32_t t = threadIdx.x, lane = t & 63, unit_cost = rule.unit_cost;
     // the workgroups of the launch share the descriptor loops; each computes the per-sequence
     // extents and range starts itself (they live in its LDS)
     const uint32_t g0 = t * ngrp + grp, GT = ngrp * T; // interleaved shares
@@ -252,6 +274,11 @@ __device__ __forceinline__ void plan_lds(uint32_t n_seqs, const uint32_t *cu, co
         // the row.
         uint32_t v[4] = {nu, nb, nr,
                          RAW && (uint64_t)p0 + nr > ((uint64_t)stride << page_shift) ? 1u : 0u};
+        // the longest unit: a sequence's last column block attends the most keys
+        uint32_t longest = nr > 0 ? unit_blocks(p0, nr) : 0u;
+#pragma unroll
+        for (int off = 32; off; off >>= 1) longest = max(longest, (uint32_t)__shfl_xor((int)longest, off));
+        if (lane == 0) w_long[t >> 6] = longest;
         block_scan_n<RAW ? 4 : 2>(v, w_s, one_wave);
         if constexpr (RAW) r0 = v[2] - nr;
         if (b < n_seqs) {
@@ -271,7 +298,28 @@ __device__ __forceinline__ void plan_lds(uint32_t n_seqs, const uint32_t *cu, co
     bool overflow = carry_units > max_units;
     if constexpr (RAW) overflow |= carry_rows != raw.n_rows || raw_bad;
     const uint32_t U = overflow ? 0 : carry_units, B = overflow ? 0 : carry_blocks;
-    const uint32_t N = min(n_wg, B);
+    // Work is split in cost: each unit's blocks are preceded by unit_cost virtual blocks (the
+    // cost of starting a unit), so a range that crosses into a unit is shorter by that much and a
+    // boundary falling in a unit's lead-in moves to the unit's start.
+    const uint64_t TC = (uint64_t)B + (uint64_t)unit_cost * U;
+    uint32_t N = min(n_wg, B);
+    bool aligned = false;
+    if (TC < (uint64_t)rule.small_cost) {
+        const uint32_t tc = (uint32_t)TC;
+        // (32-bit products: one * N < 2^18 * 13 * 2^9 on prefill, 6 * 2^11 * 8 * 2^11 on decode)
+        N = min(N, max(8u, ((tc >> rule.span_shift) + 7) & ~7u));
+        uint32_t longest = 0;
+        for (uint32_t i = 0; i < (n_seqs + 63) / 64; i++) longest = max(longest, w_long[i]);
+        uint32_t one = longest * 8, share = tc * 8, records = min(4u, (N + U) >> 7) * 8;
+        if (rule.rec) {
+            one = longest * 13;
+            if (U > rule.round_wg) one = max(one, B * 9 >> 8);
+            share = tc * (N > rule.round_wg ? 16 : 13);
+            records = (N + U) * rule.rec >> 4;
+        }
+        aligned = U && U <= n_wg && one * N <= share + records * N;
+        if (aligned) N = U;
+    }
     if (t == 0) {
         s_u0[n_seqs] = carry_units;
         s_b0[n_seqs] = carry_blocks;
@@ -291,12 +339,8 @@ __device__ __forceinline__ void plan_lds(uint32_t n_seqs, const uint32_t *cu, co
         WorkDesc d = {};
         work[w] = d;
     }
-    // Work is split in cost: each unit's blocks are preceded by unit_cost virtual blocks (the
-    // cost of starting a unit), so a range that crosses into a unit is shorter by that much and a
-    // boundary falling in a unit's lead-in moves to the unit's start.
-    const uint64_t TC = (uint64_t)B + (uint64_t)unit_cost * U;
-    const bool xcd_major = xcd && N == n_wg && N % 8 == 0;
-    const uint32_t per = N / 8;
+    const bool xcd_major = rule.xcd && N % 8 == 0;
+    const uint32_t per = N / 8, round_wg = rule.round_wg, lag = rule.lag;
     // Ranges in cost order r = 0 .. N-1 run on workgroup w(r): r itself, or XCD-major when xcd is
     // set and the grid allows (range r on workgroup (r % per) * 8 + r / per, so the workgroups of
     // one XCD - workgroup i runs on XCD i % 8 - take contiguous ranges).
@@ -315,7 +359,7 @@ __device__ __forceinline__ void plan_lds(uint32_t n_seqs, const uint32_t *cu, co
     // of 256 spans TC * w / F(N) >= TC * (256 - lag) / F(N), so with that at least 1 each start
     // lies at least one block after the previous one.  A range empty in blocks inside a unit
     // would be counted among the unit's records without writing one.
-    bool skew = lag && round_wg && round_wg < N;
+    bool skew = !aligned && lag && round_wg && round_wg < N;
     uint64_t FN = N; // the weights' sum (equal weights: one each)
     if (skew) {
         const uint64_t weighted = 256ull * N - (uint64_t)lag * late_before(N);
@@ -356,12 +400,28 @@ __device__ __forceinline__ void plan_lds(uint32_t n_seqs, const uint32_t *cu, co
 #pragma unroll 1
     for (uint32_t r0 = wave * 63; r0 < share; r0 += 63 * (T / 64)) {
         const uint32_t r = grp * share + r0 + lane;
-        const uint32_t c = r < N ? range_lo(r) : (uint32_t)TC;
         // The block at cost c, and its unit (sequence b, KV head h, column block cb): in cost,
         // sequence b starts at s_c0[b], a KV head's units span nbh + unit_cost * ncb, and a unit's
         // blocks follow its unit_cost lead-in; a cost inside a lead-in maps to the unit's first block.
         uint32_t b = 0, h = 0, cb = 0, lo = B;
-        if (r < N) {
+        uint32_t w = xcd_major ? (r % per) * 8 + r / per : r;
+        if (r < N && aligned) {
+            b = last_le(s_u0, n_seqs, r);
+            const uint32_t i = r - s_u0[b];
+            // More units than CUs: the first round's workgroups take an XCD's (or the grid's)
+            // last units in descending order, the second round's, which share their CUs, the
+            // first ones ascending, so a CU pairs a long unit of a causal chunk with a short one
+            // (2,048 rows on 4,000 keys, 8 KV heads: 195.5 us in order, 176.6 so).
+            if (N > round_wg) {
+                const uint32_t n = xcd_major ? per : N, first = xcd_major ? round_wg / 8 : round_wg;
+                const uint32_t k = xcd_major ? r % per : r, j = n - 1 - k < first ? n - 1 - k : k + first;
+                w = xcd_major ? j * 8 + r / per : j;
+            }
+            h = i / s_ncb[b];
+            cb = i - h * s_ncb[b];
+            lo = s_b0[b] + h * s_nbh[b] + cb * ((s_p0[b] + 31) / 32) + new_blocks_before(cb, rpc);
+        } else if (r < N) {
+            const uint32_t c = range_lo(r);
             b = last_le(s_c0, n_seqs, c);
             const uint32_t ncb = s_ncb[b], cblocks = (s_p0[b] + 31) / 32, nbh = s_nbh[b];
             const uint32_t hsp = nbh + unit_cost * ncb, co = c - s_c0[b];
@@ -403,7 +463,7 @@ __device__ __forceinline__ void plan_lds(uint32_t n_seqs, const uint32_t *cu, co
         }
         if (pre) d.flags |= 1;
         d.pre = make_uint4(v[0], v[1], v[2], v[3]);
-        work[xcd_major ? (r % per) * 8 + r / per : r] = d;
+        work[w] = d;
     }
     // each unit's descriptor, and its merge descriptor from it
 #pragma unroll 1
@@ -424,7 +484,7 @@ __device__ __forceinline__ void plan_lds(uint32_t n_seqs, const uint32_t *cu, co
                 wf = div_by((uint64_t)(cf + 1) * N - 1, TC, inv_tc);
                 wl = div_by((uint64_t)(cl + 1) * N - 1, TC, inv_tc);
             }
-            if (wf != wl) m = MergeDesc{wf + u, wl - wf + 1, ud.rowbeg, ud.nrows_hk};
+            if (wf != wl && !aligned) m = MergeDesc{wf + u, wl - wf + 1, ud.rowbeg, ud.nrows_hk};
         }
         merge[u] = m;
     }
@@ -433,10 +493,10 @@ __device__ __forceinline__ void plan_lds(uint32_t n_seqs, const uint32_t *cu, co
 __global__ __launch_bounds__(kPlanThreads) void plan_lds_kernel(
     uint32_t n_seqs, const uint32_t *cu, const uint32_t *positions, const uint32_t *sequences,
     const uint32_t *pages, uint32_t stride, uint32_t page_shift, uint32_t rpc, uint32_t hkv,
-    uint32_t max_units, uint32_t n_wg, uint32_t unit_cost, uint32_t round_wg, uint32_t lag,
-    uint32_t xcd, UnitDesc *units, WorkDesc *work, MergeDesc *merge, uint32_t *header) {
+    uint32_t max_units, uint32_t n_wg, PlanRule rule, UnitDesc *units, WorkDesc *work,
+    MergeDesc *merge, uint32_t *header) {
     plan_lds<false>(n_seqs, cu, positions, sequences, RawSeqs{}, pages, stride, page_shift, rpc, hkv, max_units,
-             n_wg, unit_cost, round_wg, lag, xcd, blockIdx.x, gridDim.x, units, work, merge, header);
+             n_wg, rule, blockIdx.x, gridDim.x, units, work, merge, header);
 }
 
 struct PackArgs {
@@ -455,12 +515,11 @@ constexpr uint32_t kSetupChecks = 16, kFoundWords = 16;
 // word), and the kSetupChecks after it check the block tables.
 __global__ __launch_bounds__(kPlanThreads) void pack_plan_kernel(
     uint32_t n_seqs, PackArgs pk, RawSeqs raw, uint32_t rpc, uint32_t hkv, uint32_t max_units,
-    uint32_t n_wg, uint32_t unit_cost, uint32_t round_wg, uint32_t lag, uint32_t xcd, UnitDesc *units,
-    WorkDesc *work, MergeDesc *merge, uint32_t *header) {
+    uint32_t n_wg, PlanRule rule, UnitDesc *units, WorkDesc *work, MergeDesc *merge, uint32_t *header) {
     const uint32_t bid = blockIdx.x;
     if (bid < kPlanGroups) {
         plan_lds<true>(n_seqs, nullptr, nullptr, nullptr, raw, pk.pages, pk.stride, pk.page_shift, rpc, hkv,
-                 max_units, n_wg, unit_cost, round_wg, lag, xcd, bid, kPlanGroups, units, work, merge,
+                 max_units, n_wg, rule, bid, kPlanGroups, units, work, merge,
                  header);
     } else if (bid == kPlanGroups) {
         pack_rows_block(n_seqs, pk.seq_slots, pk.q_lens, pk.cached, pk.pages, pk.stride, pk.page_shift,
@@ -2500,12 +2559,19 @@ __global__ __launch_bounds__(kCombineThreads) void combine_kernel(AttnParams p) 
 // Columns merged by one wave of combine_wide_kernel, and record passes loaded per batch.
 constexpr uint32_t kWideCombineCols = 4;
 constexpr uint32_t kWideCombinePasses = 2;
+// Units expected to hold at least kWideSomeRecords records have one column per wave merged,
+// kWideSomePasses passes at once, so that more waves share the longer lists: 512 rows on 4,000
+// keys 47.1 -> 44.4 us (8 records a unit) and 64.5 -> 61.7 (4), 32 rows on 1,000 keys 31.2 -> 21.8
+// (41).  With fewer records most of a one-column wave's loads would be past the list (two or three
+// records: 1-4 us slower); eight passes at once are slower for the same reason (32 rows of 16
+// sequences on 1,000 keys 34.6 us against 32.1), and a workgroup per column, as combine_kernel
+// merges, starts too many workgroups (54.8 us against 44.4 at 8 records).
+constexpr uint32_t kWideSomeRecords = 4, kWideSomePasses = 4;
 
 // REC: record rows normalised in f32 (0), f16 (1) or bf16 (2).
-template <int D, int REC>
+template <int D, int REC, uint32_t CW, uint32_t KP>
 __global__ __launch_bounds__(256) void combine_wide_kernel(AttnParams p) {
     constexpr uint32_t Q = D / 4, RPP = 64 / Q, COLS = 16 * kWideNTDev;
-    constexpr uint32_t CW = kWideCombineCols, KP = kWideCombinePasses;
     const uint32_t u = blockIdx.x, lane = threadIdx.x & 63;
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const uint32_t col0 = (blockIdx.y * 4 + wave) * CW; // this wave's first column
@@ -2630,6 +2696,23 @@ static hipError_t launch_combine(uint32_t split, dim3 grid, const AttnParams &p,
         return launch<combine_kernel<D, NT, 0, REC>>(g, block, 0, s, p);
     }
     return launch<combine_kernel<D, NT, 1, REC>>(grid, block, 0, s, p);
+}
+
+template <int D, int REC>
+static hipError_t launch_combine_wide_rec(uint32_t per_unit, uint32_t units, const AttnParams &p, hipStream_t s) {
+    const dim3 block(kCombineThreads);
+    if (per_unit >= kWideSomeRecords)
+        return launch<combine_wide_kernel<D, REC, 1, kWideSomePasses>>(dim3(units, 16 * kWideNT / 4), block, 0, s, p);
+    return launch<combine_wide_kernel<D, REC, kWideCombineCols, kWideCombinePasses>>(
+        dim3(units, 16 * kWideNT / (4 * kWideCombineCols)), block, 0, s, p);
+}
+
+template <int D>
+static hipError_t launch_combine_wide(int rec, uint32_t per_unit, uint32_t units, const AttnParams &p,
+                                      hipStream_t s) {
+    if (rec == 0) return launch_combine_wide_rec<D, 0>(per_unit, units, p, s);
+    if (rec == 1) return launch_combine_wide_rec<D, 1>(per_unit, units, p, s);
+    return launch_combine_wide_rec<D, 2>(per_unit, units, p, s);
 }
 
 static Layout layout_for(const lia_attention_config *c, uint32_t n_wg) {
@@ -2915,8 +2998,12 @@ static int run_stages(int stages, const lia_attention_config *c, uint32_t n_seqs
         // the config-2 step 1.3-1.4 % faster (its attention launch alone 0.15 us slower), the
         // config-3 prefill kernel 3 % faster, config 5 2 us shorter, config 4 unchanged.
         const uint32_t xcd = 1;
-        const uint32_t cost = NT == kWideNT ? kUnitCostWide : kUnitCostDecode;
-        const uint32_t lag = NT == kWideNT ? kLagWide : kLagDecode;
+        const bool wide = NT == kWideNT;
+        const uint32_t lag = wide ? kLagWide : kLagDecode;
+        const bool rec32 = p.out_f32 || c->kv_dtype == LIA_FP8_E4M3;
+        const PlanRule rule{wide ? kUnitCostWide : kUnitCostDecode, lia_device_cus(), lag, xcd,
+                            wide ? 1u << 18 : 6 * n_wg, wide ? 0u : 1u,
+                            wide ? (rec32 ? 9u : 5u) : 0u};
         // The parallel plan takes any number of workgroups (its descriptor loops stride); only its
         // weighted range starts are an LDS table of kPlanThreads.  head_dim 64 decode launches 1,536
         // workgroups (2,048 on FP8 pools): with the serial plan_kernel behind the two packing
@@ -2927,8 +3014,7 @@ static int run_stages(int stages, const lia_attention_config *c, uint32_t n_seqs
             // launch, then the step's verdict
             const RawSeqs raw{pk->q_lens, pk->cached, pk->seq_slots, n_rows};
             e = launch<pack_plan_kernel>(dim3(kPlanGroups + 1 + kSetupChecks), dim3(kPlanThreads), 0, s,
-                                         n_seqs, *pk, raw, rpc, c->num_kv_heads, L.max_units, n_wg, cost,
-                                         lia_device_cus(), lag, xcd, units, work, merge, header);
+                                         n_seqs, *pk, raw, rpc, c->num_kv_heads, L.max_units, n_wg, rule, units, work, merge, header);
             if (e == hipSuccess)
                 e = launch<setup_verdict_kernel>(dim3(1), dim3(kPlanThreads), 0, s, n_seqs, pk->max_rows,
                                                  pk->cu, pk->slot_mapping, pk->status, header, work, n_wg,
@@ -2944,12 +3030,11 @@ static int run_stages(int stages, const lia_attention_config *c, uint32_t n_seqs
             if (parallel)
             e = launch<plan_lds_kernel>(dim3(kPlanGroups), dim3(kPlanThreads), 0, s, n_seqs, cu_seqlens,
                                         positions, sequences, pages, c->stride, p.page_shift, rpc,
-                                        c->num_kv_heads, L.max_units, n_wg, cost, lia_device_cus(), lag,
-                                        xcd, units, work, merge, header);
+                                        c->num_kv_heads, L.max_units, n_wg, rule, units, work, merge, header);
             else
             e = launch<plan_kernel>(dim3(1), dim3(256), 0, s, n_seqs, cu_seqlens, positions,
                                     sequences, pages, c->stride, p.page_shift, rpc, c->num_kv_heads,
-                                    L.max_units, n_wg, xcd, units, work, merge, header);
+                                    L.max_units, n_wg, rule.xcd, units, work, merge, header);
         }
     }
     if (e == hipSuccess && (stages & kPartial)) {
@@ -3000,19 +3085,14 @@ static int run_stages(int stages, const lia_attention_config *c, uint32_t n_seqs
         else if (rec == 2) e = launch_combine<DD, NN, 2>(split, grid, p, s);                      \
         else e = launch_combine<DD, NN, 0>(split, grid, p, s);                                    \
     } while (0)
-        const dim3 wgrid(grid.x, 16 * kWideNT / (4 * kWideCombineCols));
         if (c->head_dim == 128) {
             if (NT == 1) LIA_COMBINE(128, 1);
             else if (NT == 2) LIA_COMBINE(128, 2);
-            else if (rec == 0) e = launch<combine_wide_kernel<128, 0>>(wgrid, dim3(256), 0, s, p);
-            else if (rec == 2) e = launch<combine_wide_kernel<128, 2>>(wgrid, dim3(256), 0, s, p);
-            else e = launch<combine_wide_kernel<128, 1>>(wgrid, dim3(256), 0, s, p);
+            else e = launch_combine_wide<128>(rec, per_unit, grid.x, p, s);
         } else {
             if (NT == 1) LIA_COMBINE(64, 1);
             else if (NT == 2) LIA_COMBINE(64, 2);
-            else if (rec == 0) e = launch<combine_wide_kernel<64, 0>>(wgrid, dim3(256), 0, s, p);
-            else if (rec == 2) e = launch<combine_wide_kernel<64, 2>>(wgrid, dim3(256), 0, s, p);
-            else e = launch<combine_wide_kernel<64, 1>>(wgrid, dim3(256), 0, s, p);
+            else e = launch_combine_wide<64>(rec, per_unit, grid.x, p, s);
         }
 #undef LIA_COMBINE
     }

@@ -455,3 +455,32 @@ def test_fp8_decode_large_v_scales(lia, wl):
     print(f"[case] fp8 large V scales: max_abs/scale={mx / scale:.3e} mean/scale={mean / scale:.3e}",
           flush=True)
     assert mx / scale < 5e-2 and mean / scale < 5e-3
+
+
+# label, new rows, cached keys, hq, hkv, d, pool, output, whether each unit gets one range
+RANGE_CASES = [
+    ("one unit per range, one round", [100, 97, 33, 128], [0, 0, 31, 1], 16, 2, 128, BF16, F32, True),
+    ("one unit per range, FP8", [100, 97, 33, 128], [0, 0, 31, 1], 16, 2, 128, FP8, BF16, True),
+    ("two rounds, not a multiple of 8", [600] * 7, [600, 590, 610, 601, 577, 640, 609], 8, 1, 64, BF16, BF16, True),
+    ("two full rounds", [64] * 16, list(range(200, 296, 6)), 64, 8, 64, F16, BF16, True),
+    ("split, many records", [32], [3000], 16, 2, 128, BF16, BF16, False),
+    ("split, records of two lengths, f32", [40, 17], [2500, 900], 16, 2, 128, F16, F32, False),
+    ("decode, one unit per range", [1] * 150, list(range(0, 90)) + [70] * 60, 16, 4, 128, BF16, F32, True),
+    ("decode, ranges of two blocks", [3, 3], [5000, 200], 16, 2, 128, BF16, BF16, False),
+    ("decode, one key", [1], [0], 8, 2, 64, BF16, BF16, False),
+]
+
+
+@pytest.mark.parametrize("label,new,cached,hq,hkv,d,kv,out,one", RANGE_CASES, ids=[c[0] for c in RANGE_CASES])
+def test_ranges_of_small_batches(lia, wl, label, new, cached, hq, hkv, d, kv, out, one):
+    """Batches below the size at which every workgroup gets an equal range: one range per unit (no
+    split records; in two rounds the order pairs long units with short ones) and fewer, longer
+    ranges, against the float64 oracle.  The plan's header says which it chose."""
+    g = wl.Geometry(hq=hq, hkv=hkv, d=d, kv_dtype=kv, q_dtype=BF16, out_dtype=out)
+    new, cached = np.array(new), np.array(cached)
+    case = G.Case(wl.custom(new + cached, new, geom=g, seed=len(new)), seed=len(new))
+    _check(case, lia, label)
+    units, blocks, ranges, overflow = case.last_ws[:16].view(torch.int32).tolist()
+    print(f"[case] {label}: {units} units, {blocks} blocks, {ranges} ranges", flush=True)
+    assert overflow == 0 and ranges <= max(8, blocks)
+    assert (ranges == units) if one else (ranges > units or blocks == units)
