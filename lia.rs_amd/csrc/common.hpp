@@ -78,6 +78,39 @@ __device__ __forceinline__ uint8_t f32_to_e4m3(float f) {
     return (uint8_t)(sign | code);
 }
 
+// Quotients by one divisor, for e4m3 codes: x / s as IEEE division rounds it wherever the code
+// depends on it.  From a correctly rounded reciprocal, Markstein's correction (q + (x - q s) / s
+// with a fused remainder; "Computation of elementary functions on the IBM RISC System/6000", 1990)
+// twice: the first brings q within an ulp, the second rounds it correctly: five operations, where
+// the compiler's division sequence takes eleven.  The remainders are exact for |s| in [2^-90, 2^90]
+// and quotients of at least 2^-11 (below 2^-10 every code is 0); above 1024 the code saturates
+// whatever the last bits.  Other divisors take the division.
+struct Divisor {
+    float s, inv;
+    bool plain;
+};
+__device__ __forceinline__ Divisor divisor(float s) {
+    return {s, 1.0f / s, fabsf(s) >= 0x1p-90f && fabsf(s) <= 0x1p90f};
+}
+__device__ __forceinline__ float quotient(float x, const Divisor &d) {
+    if (!d.plain) return x / d.s;
+    const float q0 = x * d.inv;
+    const float q1 = __builtin_fmaf(__builtin_fmaf(-q0, d.s, x), d.inv, q0);
+    const float q2 = __builtin_fmaf(__builtin_fmaf(-q1, d.s, x), d.inv, q1);
+    return fabsf(q0) < 1024.0f ? __builtin_copysignf(q2, q0) : q0; // (-0 keeps its sign)
+}
+
+// f32_to_e4m3 of four values, packed: the hardware conversion rounds to nearest even as it does;
+// the clamp saturates, and NaNs (0x7f whatever their sign) take the software conversion.
+__device__ __forceinline__ uint32_t f32x4_to_e4m3x4(float a, float b, float c, float d) {
+    if (__builtin_isunordered(a, b) || __builtin_isunordered(c, d))
+        return (uint32_t)f32_to_e4m3(a) | ((uint32_t)f32_to_e4m3(b) << 8) | ((uint32_t)f32_to_e4m3(c) << 16) |
+               ((uint32_t)f32_to_e4m3(d) << 24);
+    auto sat = [](float x) { return fminf(fmaxf(x, -448.0f), 448.0f); };
+    const int lo = __builtin_amdgcn_cvt_pk_fp8_f32(sat(a), sat(b), 0, false);
+    return (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(sat(c), sat(d), lo, true);
+}
+
 // Two e4m3 bytes (bits 0-7 and 16-23 of t) -> two f16 lanes holding value * 2^-8.
 // E4M3 is a sub-format of binary16 once the exponent bias is moved from 7 to 15:
 // shifting the 7 exponent+mantissa bits left by 7 yields exactly value * 2^-8 for

@@ -17,7 +17,7 @@
 namespace lia {
 
 constexpr int kMaxLaunchDevices = 64;
-constexpr int kMaxKernels = 128;
+constexpr int kMaxKernels = 256;
 
 // One cached function per (kernel, device).  `host` is the kernel's host-side handle.
 struct KernelSlot {

@@ -202,3 +202,64 @@ def test_engine_step_append_then_attend(lia, wl, O):
                           O.to_f32(q, BF16), kc, vc)
     err = np.abs(out.cpu().numpy() - ref)
     assert err.max() < 2e-2 and err.mean() < 2e-3
+
+
+def _append_plain(O, lia, hkv, d, kv, src, k, v, scales, offset=0):
+    """rows of k and v appended to slots 3, 4, .. of a 16-token-page pool, here and by the oracle;
+    offset: elements by which the source arrays start past their (aligned) allocation."""
+    rows, W, P = k.shape[0], hkv * d, 16
+    pool = -(-(rows + 3) // P)
+    store = np.uint8 if kv == FP8 else np.uint16
+    kc, vc = np.zeros(pool * P * W, store), np.full(pool * P * W, 9, store)
+    ks = vs = None
+    if kv == FP8:
+        ks, vs = np.resize(scales, pool * hkv).astype(np.float32), np.resize(scales[::-1], pool * hkv).astype(np.float32)
+    slots = np.arange(3, 3 + rows).astype(np.uint32)
+    tdt = {F32: torch.float32, F16: torch.float16, BF16: torch.bfloat16}[src]
+
+    def dev(a):
+        t = G.to_dev(np.concatenate([np.zeros(offset, a.dtype), a.reshape(-1)]))
+        return (t if src == F32 else t.view(tdt))[offset:].view(rows, W)
+
+    dkc, dvc = (G.to_dev(x.view(np.int16) if kv != FP8 else x).clone() for x in (kc, vc))
+    dks, dvs = (None, None) if ks is None else (G.to_dev(ks).clone(), G.to_dev(vs).clone())
+    with np.errstate(all="ignore"):
+        O.kv_append(O.KVLayout(hkv, d, P, pool, kv), slots, slots * 0, np.arange(pool), pool, k, v, kc, vc,
+                    src_dtype=src, slot_mapping=slots, k_scales=ks, v_scales=vs)
+    lia.kv_append(lia.KVLayout(hkv, d, P, pool, kv), dev(k), dev(v), dkc, dvc, slot_mapping=G.u32_dev(slots),
+                  k_scales=dks, v_scales=dvs)
+    torch.cuda.synchronize()
+    assert np.array_equal(dkc.cpu().numpy().view(store), kc) and np.array_equal(dvc.cpu().numpy().view(store), vc)
+    if ks is not None:
+        assert np.array_equal(dks.cpu().numpy(), ks) and np.array_equal(dvs.cpu().numpy(), vs)
+
+
+SCALES = [1.0, 0.0, 0.0078125, 3.3e-3, 448.0, 1e-30, 1e-27, 8e-28, 1e30, 1.2e27, 1e-40, -0.5, 1.0 / 448.0, 0.7]
+
+
+@pytest.mark.parametrize("kv", [F16, BF16, FP8])
+@pytest.mark.parametrize("src", [F16, BF16])
+def test_kv_append_every_16_bit_value(O, lia, kv, src):
+    """Every 16-bit pattern (NaNs, infinities, subnormals and both zeros among them) into every pool
+    type, on FP8 pools under scales at and past the ends of the fast quotient's range."""
+    k = np.resize(np.arange(65536, dtype=np.uint32), 65536).astype(np.uint16).reshape(512, 128)
+    for shift in range(0, len(SCALES) if kv == FP8 else 1, 4):
+        _append_plain(O, lia, 2, 64, kv, src, k, k[::-1].copy(), SCALES[shift:] + SCALES[:shift])
+
+
+@pytest.mark.parametrize("hkv,d,offset", [(1, 8, 0), (3, 24, 0), (2, 12, 0), (5, 4, 0), (2, 64, 1), (1, 128, 8)])
+@pytest.mark.parametrize("kv,src", [(FP8, F32), (FP8, BF16), (BF16, F32), (F16, F16)])
+def test_kv_append_edges(O, lia, hkv, d, offset, kv, src):
+    """Row widths and alignments on both sides of the vector kernel's conditions, f32 values one ulp
+    about the rounding boundaries of e4m3 quotients."""
+    rng = np.random.default_rng(hkv * 100 + d)
+    rows = 37
+    scales = rng.uniform(1e-3, 2.0, 16).astype(np.float32)
+    x = rng.standard_normal((2, rows, hkv * d)).astype(np.float32) * 100
+    if kv == FP8 and src == F32:
+        code = rng.integers(0, 1 << 12, x.shape)  # values (1 + m/16) 2^e: e4m3 values and their midpoints
+        x = (((16 + code % 16) / 16.0) * 2.0 ** (code // 16 % 16 - 9) * rng.choice(scales, x.shape)).astype(np.float32)
+        x = np.nextafter(x, np.float32(np.inf) * rng.choice([-1, 1], x.shape).astype(np.float32))
+    if src != F32:
+        x = O.from_f32(x, src)
+    _append_plain(O, lia, hkv, d, kv, src, x[0], x[1], scales, offset)
