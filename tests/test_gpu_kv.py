@@ -263,3 +263,41 @@ def test_kv_append_edges(O, lia, hkv, d, offset, kv, src):
     if src != F32:
         x = O.from_f32(x, src)
     _append_plain(O, lia, hkv, d, kv, src, x[0], x[1], scales, offset)
+
+
+@pytest.mark.parametrize("src", [F32, F16, BF16])
+@pytest.mark.parametrize("hkv,d,page,offset", [(2, 128, 16, 0), (3, 64, 16, 0), (1, 128, 64, 0), (2, 64, 128, 0),
+                                               (2, 128, 128, 0), (2, 24, 16, 0), (2, 8, 1, 0), (2, 64, 32, 1)])
+def test_kv_quantize_pages_geometries(O, lia, src, hkv, d, page, offset):
+    """Pages on both sides of the register-resident kernel's conditions (piece counts 1 to 1,024 and
+    past them, rows that are no power of two, a source off its alignment), with zero pages, an
+    infinity, NaNs, subnormal and very large pages: codes and scales bit for bit."""
+    rng = np.random.default_rng(page + d)
+    n, pool = 11, 17
+    x = rng.standard_normal((2, n, page, hkv, d)).astype(np.float32)
+    x[:, 1] = 0
+    x[0, 2] = -0.0
+    x[:, 3] *= 1e-38
+    x[:, 4] *= 3e37 if src != F16 else 1e4
+    x[0, 5, -1, 0, -1] = np.inf
+    x[1, 6, 0, 0, ::3] = np.nan
+    x[0, 7] *= 6e-8
+    with np.errstate(all="ignore"):
+        x = x if src == F32 else O.from_f32(x, src).reshape(x.shape)
+    ids = rng.permutation(pool)[:n].astype(np.uint32)
+    W = pool * page * hkv * d
+    kc, vc, ks, vs = np.zeros(W, np.uint8), np.zeros(W, np.uint8), np.zeros(pool * hkv, np.float32), np.zeros(pool * hkv, np.float32)
+    O.kv_quantize_pages(O.KVLayout(hkv, d, page, pool, FP8), ids, x[0], x[1], kc, vc, ks, vs, src_dtype=src)
+    tdt = {F32: torch.float32, F16: torch.float16, BF16: torch.bfloat16}[src]
+
+    def dev(a):
+        t = G.to_dev(np.concatenate([np.zeros(offset, a.dtype), a.reshape(-1)]))
+        return (t if src == F32 else t.view(tdt))[offset:]
+
+    got = [torch.zeros(W, dtype=torch.uint8, device="cuda") for _ in "kv"]
+    sc = [torch.zeros(pool * hkv, device="cuda") for _ in "kv"]
+    lia.kv_quantize_pages(lia.KVLayout(hkv, d, page, pool, FP8), G.u32_dev(ids), dev(x[0]), dev(x[1]), *got, *sc)
+    torch.cuda.synchronize()
+    for a, b in ((sc[0], ks), (sc[1], vs)):
+        assert np.array_equal(a.cpu().numpy().view(np.uint32), b.view(np.uint32))
+    assert np.array_equal(got[0].cpu().numpy(), kc) and np.array_equal(got[1].cpu().numpy(), vc)
