@@ -169,6 +169,141 @@ __global__ __launch_bounds__(256) void nucleus_candidates_kernel(
     if (rank < kSlots) candidates[(size_t)group * kSlots + rank] = word;
 }
 
+// One row's parts reduced for the host: the sums over its parts and its kRowWords best candidates
+// (ranks 0 .. 19 of every part) by the candidate order.  kept = 0 with candidates there means that
+// too many tie for a place; the host then reads the row's part records.
+constexpr uint32_t kRowWords = 128;   // select_nucleus's first prefix
+struct RowSummary {
+    double maximum, total;            // over the parts; total: the softmax mass at `maximum`
+    float omitted;                    // largest candidate left out of a part's 20
+    uint32_t kept, count;             // words below, candidates in all
+    uint32_t invalid;                 // some part's mass is not finite
+    uint64_t words[kRowWords];        // (id << 32 | f32 bits), best first
+};
+
+constexpr uint32_t kRowThreads = 512, kRowStage = 256;
+
+// One workgroup per row; W words of the row's records per thread.  The host's reduction reads 21
+// words of each of a row's parts (23.5 KB a row at 130,560 entries) and sorts 2,560 candidates: 64
+// rows took 27 us to copy and about 600 us of one host core.  Here: a bit-by-bit search with ballot
+// counts for a threshold that 128 to 256 candidates pass (one barrier a step, and it stops at the
+// first such threshold), then each survivor's rank among the survivors.  Bound by the search's
+// barriers and the loads before it (10.6 us for 64 rows); the copy is 1,056 bytes a row.
+template <int W>
+__global__ __launch_bounds__(kRowThreads) void nucleus_rows_kernel(
+        uint32_t parts, const double *__restrict__ temperatures, const uint64_t *__restrict__ candidates,
+        const double *__restrict__ normalizers, RowSummary *__restrict__ summaries) {
+    constexpr uint32_t WAVES = kRowThreads / 64;
+    __shared__ uint64_t s_key[kRowStage];
+    __shared__ uint32_t s_cnt[2][WAVES], s_omit[WAVES], s_bad[WAVES], s_n;
+    __shared__ double s_max[WAVES], s_sum[WAVES];
+    const uint32_t row = blockIdx.x, t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    const uint64_t *words = candidates + (size_t)row * parts * kSlots;
+    const uint32_t n_words = parts * kSlots;
+    RowSummary *out = summaries + row;
+    if (t == 0) s_n = 0;
+    uint32_t u[W], id[W], omit = 0;   // biased order keys of the finite values, 0 = none
+#pragma unroll
+    for (int c = 0; c < W; c++) {
+        const uint32_t i = c * kRowThreads + t;
+        const uint64_t w = words[min(i, n_words - 1)];
+        const uint32_t bits = (uint32_t)w;
+        id[c] = (uint32_t)(w >> 32);
+        const bool live = i < n_words && id[c] != 0xFFFFFFFFu && (bits & 0x7f800000u) != 0x7f800000u;
+        const uint32_t key = live ? (uint32_t)total_key(bits) ^ 0x80000000u : 0u;
+        const bool last = i % kSlots == kSlots - 1;
+        u[c] = last ? 0u : key;
+        omit = max(omit, last ? key : 0u);
+    }
+    double mx = -INFINITY, mass = 0.0;
+    bool bad = false;
+    if (t < parts) {
+        const double *ns = normalizers + ((size_t)row * parts + t) * 2;
+        mx = ns[0];
+        mass = ns[1];
+        bad = !isfinite(mass);
+    }
+    double m = mx;
+#pragma unroll
+    for (int o = 32; o; o >>= 1) {
+        m = fmax(m, __shfl_xor(m, o));
+        omit = max(omit, (uint32_t)__shfl_xor((int)omit, o));
+    }
+    const bool any_bad = __any(bad);
+    if (lane == 0) {
+        s_max[wave] = m;
+        s_omit[wave] = omit;
+        s_bad[wave] = any_bad;
+    }
+    // candidates with keys >= bound, over the workgroup
+    uint32_t turn = 0;
+    auto count = [&](uint32_t bound) {
+        uint32_t n = 0;
+#pragma unroll
+        for (int c = 0; c < W; c++) n += __builtin_popcountll(__ballot(u[c] >= bound));
+        if (lane == 0) s_cnt[turn][wave] = n;
+        lds_barrier();
+        n = 0;
+#pragma unroll
+        for (uint32_t w = 0; w < WAVES; w++) n += s_cnt[turn][w];
+        turn ^= 1;
+        return n;
+    };
+    const uint32_t all = count(1); // (also publishes the maxima)
+    double maximum = -INFINITY;
+#pragma unroll
+    for (uint32_t w = 0; w < WAVES; w++) maximum = fmax(maximum, s_max[w]);
+    const double temp = temperatures[row];
+    double sum = t < parts && temp > 0.0 && mass > 0.0 ? mass * exp((mx - maximum) / temp) : 0.0;
+#pragma unroll
+    for (int o = 32; o; o >>= 1) sum += __shfl_xor(sum, o);
+    if (lane == 0) s_sum[wave] = sum;
+    uint32_t bound = 1, n = all;
+    if (all > kRowStage) {
+        bound = 0;
+        for (int bit = 31; bit >= 0; bit--) { // the counts are the same in every thread
+            const uint32_t b = bound | (1u << bit);
+            const uint32_t k = count(b);
+            if (k >= kRowWords) {
+                bound = b;
+                n = k;
+                if (k <= kRowStage) break;
+            }
+        }
+    }
+    const bool fits = n <= kRowStage;
+    if (fits) {
+#pragma unroll
+        for (int c = 0; c < W; c++)
+            if (u[c] >= bound) s_key[atomicAdd(&s_n, 1u)] = (uint64_t)u[c] << 32 | id[c];
+    }
+    lds_barrier();
+    if (fits && t < n) {
+        const uint64_t mine = s_key[t];
+        uint32_t rank = 0;
+#pragma unroll 8
+        for (uint32_t k = 0; k < n; k++) rank += s_key[k] > mine;
+        if (rank < kRowWords)
+            out->words[rank] = mine << 32 | (uint32_t)total_key((uint32_t)(mine >> 32) ^ 0x80000000u);
+    }
+    if (t == 0) {
+        double total = 0.0;
+        uint32_t om = 0, inv = 0;
+#pragma unroll
+        for (uint32_t w = 0; w < WAVES; w++) {
+            total += s_sum[w];
+            om = max(om, s_omit[w]);
+            inv |= s_bad[w];
+        }
+        out->maximum = maximum;
+        out->total = total;
+        out->omitted = om ? __uint_as_float((uint32_t)total_key(om ^ 0x80000000u)) : -INFINITY;
+        out->kept = fits ? min(n, kRowWords) : 0u;
+        out->count = all;
+        out->invalid = inv;
+    }
+}
+
 // ------------------------------------------------------------------ host sampler
 
 // MT19937 and the reference sampler's two-word canonical double (src/sampling/random.rs).
@@ -374,6 +509,32 @@ struct lia_sampler {
         return 1;
     }
 
+    // checked_nucleus on the `kept` best of `count` candidates, best first: the same sums in the same
+    // order, taken only until the cutoff.  2: the cutoff lies past them.
+    int checked_nucleus_best(const uint64_t *words, uint32_t kept, uint32_t count, double maximum,
+                             double total, float omitted, std::vector<Entry> &out) const {
+        if (!std::isfinite(total) || !(total > 0.0) || !std::isfinite(maximum)) return LIA_E_NUCLEUS;
+        if (top_p == 1.0) return 0;
+        if (kept == 0) return LIA_E_EMPTY_DISTRIBUTION;
+        const double target = top_p * total;
+        double mass = 0.0, w = 0.0;
+        float last = 0.0f;
+        out.clear();
+        for (uint32_t i = 0; i < kept && !(i && mass >= target); i++) {
+            const uint32_t bits = (uint32_t)words[i];
+            memcpy(&last, &bits, 4);
+            w = weight(last, maximum);
+            mass += w;
+            out.push_back({(uint32_t)(words[i] >> 32), w});
+        }
+        if (!(mass >= target) && kept < count) return 2;
+        if (!std::isfinite(mass) || !(mass > 0.0)) return LIA_E_NUCLEUS;
+        for (Entry &e : out) e.second /= mass;
+        if (!(key_of(last) > key_of(omitted))) return 0;
+        const double uncertainty = std::fabs(total) * 1e-10;
+        return mass - w >= target - uncertainty || mass <= target + uncertainty ? 0 : 1;
+    }
+
     // Sampling::draw (src/sampling.rs:134-146).
     uint32_t draw(const std::vector<Entry> &d) {
         if (keyed) {
@@ -448,13 +609,25 @@ extern "C" int lia_sampler_draw(lia_sampler *s, uint32_t n, const uint32_t *ids,
 static uint32_t nucleus_parts(uint32_t vocab) { return (vocab + kPart - 1) / kPart; }
 static size_t align_up(size_t x, size_t a) { return (x + a - 1) / a * a; }
 
-extern "C" size_t lia_nucleus_workspace_bytes(uint32_t vocab, uint32_t rows) {
+// Bytes of the part records and temperatures of `rows` rows.
+static size_t record_bytes(uint32_t vocab, uint32_t rows) {
     const size_t g = (size_t)rows * nucleus_parts(vocab);
     return align_up(g * kSlots * 8, 256) + align_up(g * 16, 256) + align_up((size_t)rows * 8, 256);
 }
 
+// Rows whose records are reduced on the device: from 13 parts (more than two kRowWords lists: below,
+// the records are about as small as the summary), up to the words the kernel's threads hold.
+static bool summarised(uint32_t vocab) {
+    const uint32_t words = nucleus_parts(vocab) * kSlots;
+    return words > 2 * kRowWords && words <= 16 * kRowThreads;
+}
+
+extern "C" size_t lia_nucleus_workspace_bytes(uint32_t vocab, uint32_t rows) {
+    return record_bytes(vocab, rows) + (summarised(vocab) ? (size_t)rows * sizeof(RowSummary) : 0);
+}
+
 extern "C" size_t lia_nucleus_host_bytes(uint32_t vocab, uint32_t rows) {
-    return lia_nucleus_workspace_bytes(vocab, rows) + (size_t)vocab * 4;
+    return record_bytes(vocab, rows) + (size_t)vocab * 4;
 }
 
 extern "C" int lia_nucleus_candidates(uint32_t vocab, uint32_t rows, const double *temperatures,
@@ -470,71 +643,96 @@ extern "C" int lia_nucleus_candidates(uint32_t vocab, uint32_t rows, const doubl
     return e == hipSuccess ? LIA_OK : LIA_E_HIP;
 }
 
-// Workspace::read's reduction and the per-row sampling of forward_paged_sampled, on host
-// records.  `fetch_row(i, dst)` provides output row i's full logits for a fallback.
+// A row's draw from its distribution, or by the sampler's fallback on its full logits (st = 0 of a
+// nucleus row: `fetch(dst)` provides them).
 template <typename Fetch>
-static int sample_records(uint32_t vocab, uint32_t n, lia_sampler *const *samplers,
-                          const double *temps, const uint64_t *cand, const double *norm,
-                          uint32_t *tokens, uint64_t *fallbacks, Fetch fetch_row) {
+static int finish_row(uint32_t vocab, lia_sampler *s, int st, std::vector<Entry> &d, std::vector<float> &row,
+                      uint32_t *token, uint64_t *fallbacks, Fetch fetch) {
+    if (st == 0 && s->top_k == 0) {
+        if (fallbacks) ++*fallbacks;
+        row.resize(vocab);
+        st = fetch(row.data());
+        if (st == LIA_OK) st = s->distribution_logits(row.data(), vocab, d);
+    } else if (st == 1) {
+        st = LIA_OK;
+    }
+    if (st) return st;
+    *token = s->draw(d);
+    return LIA_OK;
+}
+
+// Workspace::read's reduction of one row's part records and its sampling as forward_paged_sampled
+// does it, on host records.
+template <typename Fetch>
+static int sample_parts(uint32_t vocab, lia_sampler *s, double temp, const uint64_t *cand, const double *ns,
+                        std::vector<Cand> &c, std::vector<Entry> &d, std::vector<float> &row,
+                        uint32_t *token, uint64_t *fallbacks, Fetch fetch) {
     const uint32_t parts = nucleus_parts(vocab);
-    std::vector<Cand> c;
-    std::vector<Entry> d;
-    std::vector<float> row;
-    for (uint32_t r = 0; r < n; r++) {
-        const double *ns = norm + (size_t)r * parts * 2;
-        double maximum = -INFINITY;
-        for (uint32_t p = 0; p < parts; p++) {
-            if (!std::isfinite(ns[2 * p + 1])) return LIA_E_SAMPLING_LOGITS;
-            if (ns[2 * p] > maximum) maximum = ns[2 * p];
-        }
-        double total = 0.0;
-        if (temps[r] > 0.0)
-            for (uint32_t p = 0; p < parts; p++)
-                if (ns[2 * p + 1] > 0.0) total += ns[2 * p + 1] * std::exp((ns[2 * p] - maximum) / temps[r]);
-        c.clear();
-        float omitted = -INFINITY;
-        for (uint32_t p = 0; p < parts; p++) {
-            const uint64_t *words = cand + ((size_t)r * parts + p) * kSlots;
-            for (uint32_t rank = 0; rank < kSlots; rank++) {
-                const uint32_t id = (uint32_t)(words[rank] >> 32);
-                const uint32_t bits = (uint32_t)words[rank];
-                float v;
-                memcpy(&v, &bits, 4);
-                if (id == 0xFFFFFFFFu || !std::isfinite(v)) continue;
-                if (id >= vocab) return LIA_E_NUCLEUS;
-                if (rank < kSlots - 1) c.push_back({id, v});
-                else omitted = std::max(omitted, v);
-            }
-        }
-        lia_sampler *s = samplers ? samplers[r] : nullptr;
-        if (s) {
-            int st;
-            if (s->top_k != 0) {
-                st = s->distribution(c, d);
-            } else {
-                st = s->checked_nucleus(c, maximum, total, omitted, d);
-                if (st == 0) {
-                    if (fallbacks) ++*fallbacks;
-                    row.resize(vocab);
-                    st = fetch_row(r, row.data());
-                    if (st == LIA_OK) st = s->distribution_logits(row.data(), vocab, d);
-                } else if (st == 1) {
-                    st = LIA_OK;
-                }
-            }
-            if (st) return st;
-            tokens[r] = s->draw(d);
-        } else {
-            if (c.empty()) return LIA_E_EMPTY_DISTRIBUTION;
-            Cand best = c[0];
-            for (const Cand &x : c) {
-                const int32_t k = key_of(x.second), bk = key_of(best.second);
-                if (k > bk || (k == bk && x.first > best.first)) best = x;
-            }
-            tokens[r] = best.first;
+    double maximum = -INFINITY;
+    for (uint32_t p = 0; p < parts; p++) {
+        if (!std::isfinite(ns[2 * p + 1])) return LIA_E_SAMPLING_LOGITS;
+        if (ns[2 * p] > maximum) maximum = ns[2 * p];
+    }
+    double total = 0.0;
+    if (temp > 0.0)
+        for (uint32_t p = 0; p < parts; p++)
+            if (ns[2 * p + 1] > 0.0) total += ns[2 * p + 1] * std::exp((ns[2 * p] - maximum) / temp);
+    c.clear();
+    float omitted = -INFINITY;
+    for (uint32_t p = 0; p < parts; p++) {
+        const uint64_t *words = cand + (size_t)p * kSlots;
+        for (uint32_t rank = 0; rank < kSlots; rank++) {
+            const uint32_t id = (uint32_t)(words[rank] >> 32);
+            const uint32_t bits = (uint32_t)words[rank];
+            float v;
+            memcpy(&v, &bits, 4);
+            if (id == 0xFFFFFFFFu || !std::isfinite(v)) continue;
+            if (id >= vocab) return LIA_E_NUCLEUS;
+            if (rank < kSlots - 1) c.push_back({id, v});
+            else omitted = std::max(omitted, v);
         }
     }
+    if (s) {
+        const int st = s->top_k != 0 ? s->distribution(c, d) : s->checked_nucleus(c, maximum, total, omitted, d);
+        return finish_row(vocab, s, st, d, row, token, fallbacks, fetch);
+    }
+    if (c.empty()) return LIA_E_EMPTY_DISTRIBUTION;
+    Cand best = c[0];
+    for (const Cand &x : c) {
+        const int32_t k = key_of(x.second), bk = key_of(best.second);
+        if (k > bk || (k == bk && x.first > best.first)) best = x;
+    }
+    *token = best.first;
     return LIA_OK;
+}
+
+// The same from the row's device summary.  2: it does not settle the row, the part records do.
+template <typename Fetch>
+static int sample_summary(uint32_t vocab, lia_sampler *s, const RowSummary &r, std::vector<Cand> &c,
+                          std::vector<Entry> &d, std::vector<float> &row, uint32_t *token,
+                          uint64_t *fallbacks, Fetch fetch) {
+    if (r.invalid) return LIA_E_SAMPLING_LOGITS;
+    if (r.kept == 0 && r.count) return 2;
+    if (!s) {
+        if (r.kept == 0) return LIA_E_EMPTY_DISTRIBUTION;
+        *token = (uint32_t)(r.words[0] >> 32);
+        return LIA_OK;
+    }
+    int st;
+    if (s->top_k != 0) { // at most 20: the best of all candidates are among the best kRowWords
+        c.clear();
+        for (uint32_t i = 0; i < r.kept && i < s->top_k; i++) {
+            const uint32_t bits = (uint32_t)r.words[i];
+            float v;
+            memcpy(&v, &bits, 4);
+            c.push_back({(uint32_t)(r.words[i] >> 32), v});
+        }
+        st = s->distribution(c, d);
+    } else {
+        st = s->checked_nucleus_best(r.words, r.kept, r.count, r.maximum, r.total, r.omitted, d);
+        if (st == 2) return 2;
+    }
+    return finish_row(vocab, s, st, d, row, token, fallbacks, fetch);
 }
 
 static void temperatures_for(uint32_t n, lia_sampler *const *samplers, double *t) {
@@ -553,12 +751,20 @@ extern "C" int lia_sample_host(uint32_t vocab, uint32_t n, lia_sampler *const *s
         if (samplers && samplers[i] && positions) lia_sampler_set_position(samplers[i], positions[i]);
     std::vector<double> t(n);
     temperatures_for(n, samplers, t.data());
-    return sample_records(vocab, n, samplers, t.data(), candidates, normalizers, tokens, fallbacks,
-                          [&](uint32_t r, float *dst) {
-                              if (!logits) return LIA_E_ARG;
-                              memcpy(dst, logits + (size_t)r * vocab, (size_t)vocab * 4);
-                              return LIA_OK;
-                          });
+    std::vector<Cand> c;
+    std::vector<Entry> d;
+    std::vector<float> row;
+    const size_t parts = nucleus_parts(vocab);
+    for (uint32_t r = 0; r < n; r++) {
+        const int st = sample_parts(vocab, samplers ? samplers[r] : nullptr, t[r], candidates + r * parts * kSlots,
+                                    normalizers + r * parts * 2, c, d, row, tokens + r, fallbacks, [&](float *dst) {
+                                        if (!logits) return LIA_E_ARG;
+                                        memcpy(dst, logits + (size_t)r * vocab, (size_t)vocab * 4);
+                                        return LIA_OK;
+                                    });
+        if (st) return st;
+    }
+    return LIA_OK;
 }
 
 extern "C" int lia_sample_paged(uint32_t vocab, uint32_t n, lia_sampler *const *samplers,
@@ -567,17 +773,18 @@ extern "C" int lia_sample_paged(uint32_t vocab, uint32_t n, lia_sampler *const *
                                 uint32_t *tokens, uint64_t *fallbacks, lia_stream_t stream) {
     if (vocab == 0 || !tokens || !logits || !workspace || !host) return LIA_E_ARG;
     if (n == 0) return LIA_OK;
-    if (workspace_bytes < lia_nucleus_workspace_bytes(vocab, n) ||
-        host_bytes < lia_nucleus_host_bytes(vocab, n))
-        return LIA_E_WORKSPACE;
-    const size_t g = (size_t)n * nucleus_parts(vocab);
+    const size_t records = record_bytes(vocab, n), parts = nucleus_parts(vocab);
+    if (workspace_bytes < records || host_bytes < lia_nucleus_host_bytes(vocab, n)) return LIA_E_WORKSPACE;
+    const size_t g = (size_t)n * parts;
     const size_t cand_bytes = align_up(g * kSlots * 8, 256), norm_bytes = align_up(g * 16, 256);
     uint8_t *ws = (uint8_t *)workspace, *hb = (uint8_t *)host;
     uint64_t *cand = (uint64_t *)ws;
     double *norm = (double *)(ws + cand_bytes);
     double *temps = (double *)(ws + cand_bytes + norm_bytes);
     double *htemps = (double *)(hb + cand_bytes + norm_bytes);
-    float *hrow = (float *)(hb + lia_nucleus_workspace_bytes(vocab, n));
+    float *hrow = (float *)(hb + records);
+    RowSummary *sums = (RowSummary *)(ws + records);
+    const bool summed = summarised(vocab) && workspace_bytes >= lia_nucleus_workspace_bytes(vocab, n);
     for (uint32_t i = 0; i < n; i++)
         if (samplers && samplers[i] && positions) lia_sampler_set_position(samplers[i], positions[i]);
     temperatures_for(n, samplers, htemps);
@@ -589,17 +796,51 @@ extern "C" int lia_sample_paged(uint32_t vocab, uint32_t n, lia_sampler *const *
         (void)hipStreamSynchronize(s);
         return st;
     }
-    if (hipMemcpyAsync(hb, ws, cand_bytes + norm_bytes, hipMemcpyDeviceToHost, s) != hipSuccess ||
+    // the rows' summaries down (they fit where the records would go), or every part record
+    if (summed) {
+        const hipError_t e =
+            parts * kSlots <= 8 * kRowThreads
+                ? launch<nucleus_rows_kernel<8>>(dim3(n), dim3(kRowThreads), 0, s, (uint32_t)parts, temps, cand, norm, sums)
+                : launch<nucleus_rows_kernel<16>>(dim3(n), dim3(kRowThreads), 0, s, (uint32_t)parts, temps, cand, norm, sums);
+        if (e != hipSuccess) {
+            (void)hipStreamSynchronize(s);
+            return LIA_E_HIP;
+        }
+    }
+    if (hipMemcpyAsync(hb, summed ? (const void *)sums : ws, summed ? n * sizeof(RowSummary) : cand_bytes + norm_bytes,
+                       hipMemcpyDeviceToHost, s) != hipSuccess ||
         hipStreamSynchronize(s) != hipSuccess)
         return LIA_E_HIP;
-    return sample_records(vocab, n, samplers, htemps, (const uint64_t *)hb,
-                          (const double *)(hb + cand_bytes), tokens, fallbacks,
-                          [&](uint32_t r, float *dst) {
-                              if (hipMemcpyAsync(hrow, logits + (size_t)r * vocab, (size_t)vocab * 4,
-                                                 hipMemcpyDeviceToHost, s) != hipSuccess ||
-                                  hipStreamSynchronize(s) != hipSuccess)
-                                  return LIA_E_HIP;
-                              memcpy(dst, hrow, (size_t)vocab * 4);
-                              return LIA_OK;
-                          });
+    auto down = [&](void *dst, const void *src, size_t bytes) {
+        return hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s) == hipSuccess &&
+               hipStreamSynchronize(s) == hipSuccess;
+    };
+    std::vector<Cand> c;
+    std::vector<Entry> d;
+    std::vector<float> row;
+    for (uint32_t r = 0; r < n; r++) {
+        auto fetch = [&](float *dst) {
+            if (!down(hrow, logits + (size_t)r * vocab, (size_t)vocab * 4)) return (int)LIA_E_HIP;
+            memcpy(dst, hrow, (size_t)vocab * 4);
+            return (int)LIA_OK;
+        };
+        lia_sampler *sp = samplers ? samplers[r] : nullptr;
+        int st = 2;
+        if (summed) st = sample_summary(vocab, sp, ((const RowSummary *)hb)[r], c, d, row, tokens + r, fallbacks, fetch);
+        if (st == 2) {
+            const uint64_t *rc = (const uint64_t *)hb + r * parts * kSlots;
+            const double *rn = (const double *)(hb + cand_bytes) + r * parts * 2;
+            if (summed) { // this row's records, through the full-row buffer (4 KB a part)
+                uint64_t *hc = (uint64_t *)hrow;
+                double *hn = (double *)(hc + parts * kSlots);
+                if (!down(hc, cand + r * parts * kSlots, parts * kSlots * 8) || !down(hn, norm + r * parts * 2, parts * 16))
+                    return LIA_E_HIP;
+                rc = hc;
+                rn = hn;
+            }
+            st = sample_parts(vocab, sp, htemps[r], rc, rn, c, d, row, tokens + r, fallbacks, fetch);
+        }
+        if (st) return st;
+    }
+    return LIA_OK;
 }

@@ -99,3 +99,66 @@ def test_sample_paged_mixed_samplers_match_oracle(lia):
                                               for c in configs], positions)
     assert got == want and ps.fallbacks == fallbacks
     assert got[0] == 5009
+
+
+def _edge_rows(rng, vocab):
+    """Rows whose candidates end a summary's cases: peaked, flat, all tied, nearly empty, cut inside
+    and past the first 128 candidates, and zeros of both signs among the best."""
+    x = (rng.standard_normal((9, vocab)) * 1.5).astype(np.float32)
+    x[0, rng.integers(0, vocab, 40)] += 12.0
+    x[1] *= 0.01                                       # flat: no sparse proof, full-row fallback
+    x[2] = 1.25                                        # every candidate tied
+    x[3] = -np.inf
+    x[3, [5, vocab - 1]] = [0.5, 0.25]                 # two candidates in all
+    x[4, rng.choice(vocab, 300, replace=False)] = 9.0 + rng.random(300).astype(np.float32)  # past 128
+    x[5, rng.choice(vocab, 100, replace=False)] = 14.0 + rng.random(100).astype(np.float32)
+    x[6] = np.where(rng.random(vocab) < 0.5, np.float32(0.0), np.float32(-0.0))
+    x[7] = -np.inf
+    x[7, 17] = -3.0                                    # one candidate
+    x[8, :140] = np.linspace(20, 19, 140, dtype=np.float32)  # one part's best alone
+    return x
+
+
+@pytest.mark.parametrize("vocab", [12288, 12289, 195 * 1024, 195 * 1024 + 1, 390 * 1024, 390 * 1024 + 1, 130560])
+def test_summaries_sample_as_the_records_do(lia, vocab):
+    """lia_sample_paged reduces the records on the device from 13 parts up to 390: its tokens, errors
+    and fallback count equal lia_sample_host's on the same rows' records, for greedy, top-k and
+    nucleus rows, at both sides of each limit."""
+    rng = np.random.default_rng(vocab)
+    x = _edge_rows(rng, vocab)
+    rows = x.shape[0]
+    print(f"[case] summaries vocab={vocab}", flush=True)
+    dev = torch.from_numpy(x).cuda()
+    for temp, top_k, top_p in ((0.8, 0, 0.9), (1.3, 0, 0.999), (0.7, 20, 1.0), (1.0, 3, 0.5), (1.0, 0, 1.0)):
+        make = lambda: [lia.Sampler(temp, top_k, top_p, 7 + i, position_keyed=i % 2 == 0) for i in range(rows)]  # noqa: E731
+        positions = [11 * i for i in range(rows)]
+        cand, norm = _records(lia, x, [temp if top_k == 0 else 0.0] * rows)
+        want, fb = lia.sample_host(vocab, make(), positions, cand, norm, logits=x)
+        p = lia.PagedSampler(vocab, rows)
+        p.workspace.fill_(0x7E)
+        assert p.sample(dev, make(), positions) == want, (temp, top_k, top_p)
+        assert p.fallbacks == fb
+    greedy, _ = lia.sample_host(vocab, [None] * rows, positions, *_records(lia, x, [0.0] * rows))
+    assert lia.PagedSampler(vocab, rows).sample(dev, [None] * rows, positions) == greedy
+
+
+@pytest.mark.parametrize("value,status", [(np.nan, -26), (np.inf, -26), (-np.inf, -27)])
+def test_summaries_report_the_records_errors(lia, value, status):
+    """A NaN or +inf anywhere in a row, and a row without a finite entry, fail as they do from the
+    records, at the first such row; the rows before it have been sampled."""
+    vocab = 20000
+    x = np.random.default_rng(3).standard_normal((3, vocab)).astype(np.float32)
+    if value == -np.inf:
+        x[1] = value
+    else:
+        x[1, 19999] = value
+    for samplers in ([lia.Sampler(1.0, 0, 0.9, 1) for _ in range(3)], [lia.Sampler(1.0, 5, 1.0, 1) for _ in range(3)], [None] * 3):
+        nucleus = samplers[0] is not None and samplers[0].top_k == 0
+        cand, norm = _records(lia, x, [1.0 if nucleus else 0.0] * 3)
+        with pytest.raises(lia.LiaError) as host:
+            lia.sample_host(vocab, samplers, [0] * 3, cand, norm, logits=x)
+        with pytest.raises(lia.LiaError) as dev:
+            lia.PagedSampler(vocab, 3).sample(torch.from_numpy(x).cuda(), samplers, [0] * 3)
+        assert dev.value.status == host.value.status
+        if not (value == -np.inf and nucleus):
+            assert dev.value.status == status
