@@ -2,9 +2,8 @@
 // sampler of Engine::forward_paged_sampled (src/inference/paged_sampling.rs:7-76).
 //
 // The kernel (llama_nucleus_candidates, src/gpu/kernels/llama_nucleus.rs:18-117) gives one
-// wavefront to each (row, part of 1024 vocabulary entries): lane l holds entries
-// part*1024 + l + 64j (j < 16), so every load instruction reads 256 contiguous bytes.  It
-// writes the part's 21 largest entries by the total order of their f32 bits (ties: larger
+// wavefront to each (row, part of 1024 vocabulary entries), whose load instructions read 1 KB
+// each.  It writes the part's 21 largest entries by the total order of their f32 bits (ties: larger
 // id first) as (id << 32 | bits) words, then the part's maximum and the f64 softmax mass
 // sum exp((x - max) / T) (NaN when the part holds a NaN or +inf).  The host reduces the
 // parts to one candidate list per row (src/gpu/nucleus.rs:103-143) and samples it: top-k
@@ -61,7 +60,7 @@ __global__ __launch_bounds__(256) void nucleus_candidates_kernel(
         uint32_t vocab, uint32_t parts, uint32_t groups, const double *__restrict__ temperatures,
         const float *__restrict__ logits, uint64_t *__restrict__ candidates,
         double *__restrict__ normalizers) {
-    __shared__ uint32_t stage_u[4][64], stage_off[4][64];
+    __shared__ uint64_t stage[4][64];
     const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const uint32_t group = blockIdx.x * 4 + wave;
     if (group >= groups) return;                       // whole waves leave together
@@ -69,18 +68,23 @@ __global__ __launch_bounds__(256) void nucleus_candidates_kernel(
     const uint32_t base = part * kPart;
     const uint32_t live = min(vocab - base, kPart);
     // Bounded loads: entries past the part's live range read as 0 without touching memory,
-    // so all 16 loads are issued back to back with no branch.
+    // so the loads are issued back to back with no branch.  Register j holds entry
+    // 256 (j / 4) + 4 lane + j % 4 of the part: 16 bytes a lane and load.
     const auto rsrc = make_rsrc(logits + (size_t)row * vocab + base, live * 4);
+    auto entry = [&](uint32_t j) { return 256 * (j / 4) + 4 * lane + j % 4; };
     float v[kPerLane];
 #pragma unroll
-    for (uint32_t j = 0; j < kPerLane; j++)
-        v[j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsrc, (int)((lane + 64 * j) * 4), 0, 0));
+    for (uint32_t j = 0; j < kPerLane; j += 4) {
+        const f32x4 x = __builtin_bit_cast(f32x4, buffer_load16(rsrc, entry(j) * 4));
+#pragma unroll
+        for (uint32_t i = 0; i < 4; i++) v[j + i] = x[i];
+    }
     float mx = -INFINITY;
     bool invalid = false;
     uint32_t u[kPerLane];                               // biased order keys, 0 = not visible
 #pragma unroll
     for (uint32_t j = 0; j < kPerLane; j++) {
-        const bool in = lane + 64 * j < live;
+        const bool in = entry(j) < live;
         v[j] = in ? v[j] : -INFINITY;
         mx = fmaxf(mx, v[j]);                           // ignores NaN, as f32::max does
         invalid |= in && ((v[j] != v[j]) || v[j] == INFINITY);
@@ -131,23 +135,24 @@ __global__ __launch_bounds__(256) void nucleus_candidates_kernel(
             const uint32_t r = kSlots - wave_count([&](uint32_t j) { return u[j] > T; });
             for (int bit = 9; bit >= 0; bit--) {        // the r largest offsets among u == T
                 const uint32_t c = I | (1u << bit);
-                if (wave_count([&](uint32_t j) { return u[j] == T && lane + 64 * j >= c; }) >= r) I = c;
+                if (wave_count([&](uint32_t j) { return u[j] == T && entry(j) >= c; }) >= r) I = c;
             }
             lo = T;
         }
     }
-    // compact the n_sel selected entries into LDS (any order), then rank them
+    // compact the n_sel selected entries into LDS (any order), then rank them: key << 32 | offset
+    // orders them, slots past n_sel hold 0 and rank below, so the reads go out eight at a time
+    stage[wave][lane] = 0;
     uint32_t at = 0;
 #pragma unroll
     for (uint32_t j = 0; j < kPerLane; j++) {
-        const uint32_t off = lane + 64 * j;
+        const uint32_t off = entry(j);
         const bool sel = k && (u[j] > lo || (u[j] == lo && off >= I));
         const uint64_t m = __ballot(sel);
         if (sel) {
             const uint32_t pos = at + __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
                                                                __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0));
-            stage_u[wave][pos] = u[j];
-            stage_off[wave][pos] = off;
+            stage[wave][pos] = (uint64_t)u[j] << 32 | off;
         }
         at += __builtin_popcountll(m);
     }
@@ -157,14 +162,14 @@ __global__ __launch_bounds__(256) void nucleus_candidates_kernel(
     uint64_t word = (uint64_t)0xFFFFFFFFu << 32 | __float_as_uint(-INFINITY);
     uint32_t rank = lane;                               // lanes k..20: empty slots
     if (lane < n_sel) {
-        const uint32_t mu = stage_u[wave][lane], mo = stage_off[wave][lane];
+        const uint64_t mine = stage[wave][lane];
         rank = 0;
-        for (uint32_t m = 0; m < n_sel; m++) {
-            const uint32_t ou = stage_u[wave][m], oo = stage_off[wave][m];
-            rank += ou > mu || (ou == mu && oo > mo);
+        for (uint32_t m = 0; m < n_sel; m += 8) {
+#pragma unroll
+            for (uint32_t i = 0; i < 8; i++) rank += stage[wave][m + i] > mine;
         }
-        const uint32_t bits = (uint32_t)total_key(mu ^ 0x80000000u);   // the key map is an involution
-        word = (uint64_t)(base + mo) << 32 | bits;
+        const uint32_t bits = (uint32_t)total_key((uint32_t)(mine >> 32) ^ 0x80000000u); // the key map is an involution
+        word = (uint64_t)(base + (uint32_t)mine) << 32 | bits;
     }
     if (rank < kSlots) candidates[(size_t)group * kSlots + rank] = word;
 }
