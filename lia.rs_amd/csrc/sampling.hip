@@ -48,8 +48,8 @@ __device__ __forceinline__ uint32_t wave_count(Pred pred) {
 
 // One wavefront per (row, part).  The k = min(21, visible) best entries are found without
 // k serial argmax rounds (keys biased to unsigned: u = key ^ 0x80000000):
-//  - the 21st largest lane maximum tau is a lower bound of the 21st largest entry (the 21
-//    largest lane maxima are 21 distinct entries), so the entries >= tau - usually a few
+//  - a tau that 21 lane maxima reach is a lower bound of the 21st largest entry (those maxima
+//    are 21 distinct entries), so the entries >= tau - usually a few
 //    dozen - contain the answer: when at most 64 survive they are ranked directly;
 //  - otherwise (mass ties) a bit-by-bit search with ballot counts finds the k-th largest key
 //    T, and a second search over the in-part offset settles ties at T (larger ids first).
@@ -79,25 +79,49 @@ __global__ __launch_bounds__(256) void nucleus_candidates_kernel(
 #pragma unroll
         for (uint32_t i = 0; i < 4; i++) v[j + i] = x[i];
     }
-    float mx = -INFINITY;
-    bool invalid = false;
-    uint32_t u[kPerLane];                               // biased order keys, 0 = not visible
+    // Biased order keys u (0 = not visible), and from their extremes what most parts need: the
+    // maximum, that no entry is NaN or +inf, that every entry is visible.  Keys order -inf above the
+    // negative NaNs and +inf below the positive ones.
+    constexpr uint32_t kNegInf = 0x007fffffu, kPosInf = 0xff800000u;
+    uint32_t u[kPerLane], hi = 0, least = 0xffffffffu;
 #pragma unroll
     for (uint32_t j = 0; j < kPerLane; j++) {
-        const bool in = entry(j) < live;
-        v[j] = in ? v[j] : -INFINITY;
-        mx = fmaxf(mx, v[j]);                           // ignores NaN, as f32::max does
-        invalid |= in && ((v[j] != v[j]) || v[j] == INFINITY);
-        u[j] = in ? (uint32_t)total_key(__float_as_uint(v[j])) ^ 0x80000000u : 0u;
+        const uint32_t s = __float_as_uint(v[j]);
+        u[j] = s ^ ((uint32_t)((int32_t)s >> 31) | 0x80000000u);
+        if (live < kPart && entry(j) >= live) u[j] = 0; // (live is uniform)
+        hi = max(hi, u[j]);
+        least = min(least, u[j]);
+    }
+    float mx = -INFINITY;
+    bool invalid = false;
+    const bool ordinary = !__any(hi >= kPosInf || least < kNegInf); // the whole part, no NaN, no +inf
+    if (ordinary) {
+        mx = __uint_as_float((uint32_t)total_key(hi ^ 0x80000000u));
+    } else {
+#pragma unroll
+        for (uint32_t j = 0; j < kPerLane; j++) {
+            const bool in = entry(j) < live;
+            v[j] = in ? v[j] : -INFINITY;
+            mx = fmaxf(mx, v[j]);                       // ignores NaN, as f32::max does
+            invalid |= in && ((v[j] != v[j]) || v[j] == INFINITY);
+        }
     }
 #pragma unroll
     for (int o = 32; o; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
     double sum = 0.0;
     const double t = temperatures[row];
     if (t > 0.0 && isfinite(mx)) {
+        // Quotients by the row's temperature from its reciprocal, corrected by a fused remainder:
+        // five operations, where the division sequence takes eleven.  Both sides are scaled to a
+        // temperature in [0.5, 1), and quotients below -1e6 (whose exponential is 0) cut, so no
+        // step leaves the exponent range.
+        int e2;
+        const double ts = __builtin_frexp(t, &e2), inv = 1.0 / ts;
 #pragma unroll
         for (uint32_t j = 0; j < kPerLane; j++) {
-            const double e = exp(((double)v[j] - (double)mx) / t);
+            const double x = fmax(__builtin_ldexp((double)v[j] - (double)mx, -e2), -1e6);
+            const double q = x * inv;
+            const double e = exp(__builtin_fma(__builtin_fma(-q, ts, x), inv, q));
             sum += isfinite(v[j]) ? e : 0.0;
         }
     }
@@ -109,18 +133,18 @@ __global__ __launch_bounds__(256) void nucleus_candidates_kernel(
         normalizers[2 * (size_t)group + 1] = sum;
     }
 
-    const uint32_t visible = wave_count([&](uint32_t j) { return u[j] != 0; });
+    const uint32_t visible = ordinary ? kPart : wave_count([&](uint32_t j) { return u[j] != 0; });
     const uint32_t k = min(visible, kSlots);
     // selection: u >= lo, and at u == lo only offsets >= I
     uint32_t lo = 1, I = 0, n_sel = k;
     if (k == kSlots) {
-        uint32_t lm = 0;
-#pragma unroll
-        for (uint32_t j = 0; j < kPerLane; j++) lm = max(lm, u[j]);
-        uint32_t tau = 0;                               // 21st largest lane maximum
+        // a bound that at least 21 lane maxima reach, and at most a few more
+        uint32_t tau = 0;
         for (int bit = 31; bit >= 0; bit--) {
             const uint32_t c = tau | (1u << bit);
-            if ((uint32_t)__builtin_popcountll(__ballot(lm >= c)) >= kSlots) tau = c;
+            const uint32_t n = (uint32_t)__builtin_popcountll(__ballot(hi >= c));
+            if (n >= kSlots) tau = c;
+            if (n >= kSlots && n <= kSlots + 4) break;
         }
         const uint32_t n_s = tau ? wave_count([&](uint32_t j) { return u[j] >= tau; }) : 1024u;
         if (n_s <= 64) {

@@ -162,3 +162,13 @@ def test_summaries_report_the_records_errors(lia, value, status):
         assert dev.value.status == host.value.status
         if not (value == -np.inf and nucleus):
             assert dev.value.status == status
+
+
+@pytest.mark.parametrize("temp", [1e-300, 1e-30, 0.01, 0.7, 3.0, 1e30, 1e300])
+def test_part_masses_over_the_temperature_range(lia, temp):
+    """The parts' masses against the oracle's to 1e-12 at ordinary and extreme temperatures, with
+    -inf entries and a part whose values span the f32 range."""
+    x = (np.random.default_rng(5).standard_normal((2, 3000)) * 4).astype(np.float32)
+    x[0, ::7] = -np.inf
+    x[1, :1024] *= 1e37
+    _check_records(lia, x, [temp, temp], f"temperature {temp}")
