@@ -2553,12 +2553,15 @@ __global__ __launch_bounds__(kCombineThreads) void combine_kernel(AttnParams p) 
 }
 
 // Merge for the prefill kernel's 128-column units, which are split over few workgroups
-// (2-3 records each): one wave per column, four columns per workgroup.  Lanes hold a
-// record's row as float4 quads (64 / (D/4) records per pass); the record groups are summed
-// with lane shuffles.  Same merge rule as combine_kernel.
-// Columns merged by one wave of combine_wide_kernel, and record passes loaded per batch.
+// (2-3 records each): a wave merges kWideCombineCols columns.  Lanes hold a record's row as
+// float4 quads (64 / (D/4) records per pass); as in combine_kernel each record group merges its
+// records against its own maximum and the groups merge once, at the end, by lane shuffles.  Bound by
+// the trips to memory of its short waves, so what keeps more of them resident counts: a maximum over
+// the wave and two passes loaded at once (half of them past the end of a two-record list) took 20.0
+// us for a unit list of 512 split bf16 and 22.5 for one of f32 units, this form 14.5 and 15.6 (a
+// 4,358-row step 246.8 -> 242.0 us); two columns a wave measure the same, eight 3 % slower steps.
 constexpr uint32_t kWideCombineCols = 4;
-constexpr uint32_t kWideCombinePasses = 2;
+constexpr uint32_t kWideCombinePasses = 1;
 // Units expected to hold at least kWideSomeRecords records have one column per wave merged,
 // kWideSomePasses passes at once, so that more waves share the longer lists: 512 rows on 4,000
 // keys 47.1 -> 44.4 us (8 records a unit) and 64.5 -> 61.7 (4), 32 rows on 1,000 keys 31.2 -> 21.8
@@ -2617,20 +2620,17 @@ __global__ __launch_bounds__(256) void combine_wide_kernel(AttnParams p) {
                 m[c][k] = ml.x;
                 l[c][k] = r < n ? ml.y : 0.0f;
             }
+        // each record group against its own maximum; the groups merge at the end
 #pragma unroll
         for (uint32_t c = 0; c < CW; c++) {
-            float bm = -INFINITY;
+            float nm = M[c];
 #pragma unroll
             for (uint32_t k = 0; k < KP; k++)
-                if (l[c][k] > 0.0f) bm = fmaxf(bm, m[c][k]);
-            bm = wave_max(bm);
-            const float nm = fmaxf(M[c], bm);
-            if (nm != M[c]) {
-                const float f = M[c] == -INFINITY ? 0.0f : fast_exp2(M[c] - nm);
-                num[c].x *= f; num[c].y *= f; num[c].z *= f; num[c].w *= f;
-                den[c] *= f;
-                M[c] = nm;
-            }
+                if (l[c][k] > 0.0f) nm = fmaxf(nm, m[c][k]);
+            const float f = M[c] == -INFINITY ? 0.0f : fast_exp2(M[c] - nm);
+            num[c].x *= f; num[c].y *= f; num[c].z *= f; num[c].w *= f;
+            den[c] *= f;
+            M[c] = nm;
 #pragma unroll
             for (uint32_t k = 0; k < KP; k++) {
                 const float w = l[c][k] > 0.0f ? fast_exp2(m[c][k] - M[c]) * l[c][k] : 0.0f;
@@ -2646,14 +2646,18 @@ __global__ __launch_bounds__(256) void combine_wide_kernel(AttnParams p) {
     for (uint32_t c = 0; c < CW; c++) {
         const uint32_t col = col0 + c;
         float4 x = num[c];
-        float dn = den[c];
+        float dn = den[c], mg = M[c];
 #pragma unroll
-        for (uint32_t off = Q; off < 64; off <<= 1) {
-            x.x += shfl_xor(x.x, off);
-            x.y += shfl_xor(x.y, off);
-            x.z += shfl_xor(x.z, off);
-            x.w += shfl_xor(x.w, off);
-            dn += shfl_xor(dn, off);
+        for (uint32_t off = Q; off < 64; off <<= 1) { // (a group without records holds -inf and zeros)
+            const float mo = shfl_xor(mg, off), nm = fmaxf(mg, mo);
+            const float a = mg == -INFINITY ? 0.0f : fast_exp2(mg - nm);
+            const float b = mo == -INFINITY ? 0.0f : fast_exp2(mo - nm);
+            x.x = x.x * a + shfl_xor(x.x, off) * b;
+            x.y = x.y * a + shfl_xor(x.y, off) * b;
+            x.z = x.z * a + shfl_xor(x.z, off) * b;
+            x.w = x.w * a + shfl_xor(x.w, off) * b;
+            dn = dn * a + shfl_xor(dn, off) * b;
+            mg = nm;
         }
         if (rg != 0 || col >= ncols) continue;
         const float inv = dn > 0.0f ? 1.0f / dn : 0.0f;
