@@ -254,10 +254,24 @@ def _dptr(t):
     return C.c_void_p(t.data_ptr())
 
 
+_raw_stream = None
+
+
 def _stream(stream=None):
-    import torch
-    s = stream if stream is not None else torch.cuda.current_stream()
-    return C.c_void_p(s.cuda_stream)
+    """Handle of `stream`, or of the current device's current stream.  Every launch asks for it:
+    torch's raw getter takes 0.3 us where building a Stream object took 3.2, of a launch's 8."""
+    global _raw_stream
+    if stream is not None:
+        return C.c_void_p(stream.cuda_stream)
+    if _raw_stream is None:
+        import torch
+        torch.cuda.current_stream()  # initialises the runtime; raises where there is no device
+        get, device = (getattr(torch._C, n, None) for n in ("_cuda_getCurrentRawStream", "_cuda_getDevice"))
+        if get is not None and device is not None:
+            _raw_stream = lambda: get(device())  # noqa: E731
+        else:
+            _raw_stream = lambda: torch.cuda.current_stream().cuda_stream  # noqa: E731
+    return C.c_void_p(_raw_stream())
 
 
 def torch_dtype_code(dt):
