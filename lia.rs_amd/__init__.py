@@ -909,7 +909,8 @@ class Engine:
         torch.cuda.synchronize()
 
     def stage(self, rows, tables, outputs=()):
-        """Host packing + metadata upload of Engine::run_paged (paging.rs:118-237)."""
+        """Host packing + metadata upload of Engine::run_paged (paging.rs:118-237), and the plan
+        attention() works from: the engine's workspace is the step's until its last layer."""
         import torch
         if self.paging is None:
             raise LiaError(-19, "paging is not configured")
@@ -924,26 +925,41 @@ class Engine:
         w["pages"].copy_(as_i32(packed["flat"]))
         w["cu_seqlens"][:ng + 1].copy_(as_i32(packed["cu_seqlens"]))
         w["n_seqs"], w["n_rows"] = ng, n
+        # the step's work list, the same for every layer
+        attention_plan(self.config, ng, n, w["cu_seqlens"], w["positions"], w["sequences"],
+                       w["workspace"], w["pages"])
         torch.cuda.current_stream().synchronize()
         return packed
 
     def attention(self, layer, q, k, v, out=None):
-        """Append this step's K/V rows to layer's pool and attend (llama.rs:203-288)."""
+        """Append this step's K/V rows to layer's pool and attend (llama.rs:203-288), on the plan
+        stage() made.  Rows of the pool's type (bf16 on an FP8 pool) are appended by the attention
+        call itself, others by a launch before it: two or three launches a layer where append,
+        plan, attention and combine were four."""
         import torch
         w = self.paging
         n = w["n_rows"]
         if q.shape[0] != n or k.shape[0] != n:
             raise LiaError(-20, "attention: row count differs from the staged batch")
-        layout = KVLayout(self.hkv, self.d, self.page_size, self.pool_pages, self.kv_dtype)
-        kv_append(layout, k.reshape(n, -1), v.reshape(n, -1), self.k[layer], self.v[layer],
-                  slot_mapping=w["slot_mapping"], k_scales=self.k_scales[layer],
-                  v_scales=self.v_scales[layer])
         if out is None:
             odt = torch.float32 if self.out_dtype == F32 else torch.bfloat16
             out = torch.empty((n, self.hq, self.d), dtype=odt, device=q.device)
-        paged_attention(self.config, w["n_seqs"], w["cu_seqlens"], w["positions"],
-                        w["sequences"], w["pages"], q, self.k[layer], self.v[layer], out,
-                        w["workspace"], self.k_scales[layer], self.v_scales[layer])
+        k, v, kc, vc = k.reshape(n, -1), v.reshape(n, -1), self.k[layer], self.v[layer]
+        ks, vs = self.k_scales[layer], self.v_scales[layer]
+        fp8 = self.kv_dtype == FP8
+        args = self.config, w["n_seqs"], w["pages"]
+        fused = (k.dtype == v.dtype and torch_dtype_code(k.dtype) == (BF16 if fp8 else self.kv_dtype)
+                 and (k.data_ptr() | v.data_ptr()) % 16 == 0)
+        if fused and fp8:
+            attention_partial_append_fp8(*args, w["slot_mapping"], q, k, v, kc, vc, ks, vs, out,
+                                         w["workspace"])
+        elif fused:
+            attention_partial_append(*args, w["slot_mapping"], q, k, v, kc, vc, out, w["workspace"])
+        else:
+            layout = KVLayout(self.hkv, self.d, self.page_size, self.pool_pages, self.kv_dtype)
+            kv_append(layout, k, v, kc, vc, slot_mapping=w["slot_mapping"], k_scales=ks, v_scales=vs)
+            attention_partial(*args, q, kc, vc, out, w["workspace"], ks, vs)
+        attention_merge(self.config, w["n_seqs"], n, out, w["workspace"])
         return out
 
     def _transfer(self):

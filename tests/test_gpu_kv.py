@@ -301,3 +301,55 @@ def test_kv_quantize_pages_geometries(O, lia, src, hkv, d, page, offset):
     for a, b in ((sc[0], ks), (sc[1], vs)):
         assert np.array_equal(a.cpu().numpy().view(np.uint32), b.view(np.uint32))
     assert np.array_equal(got[0].cpu().numpy(), kc) and np.array_equal(got[1].cpu().numpy(), vc)
+
+
+@pytest.mark.parametrize("kv", [F16, BF16, FP8])
+@pytest.mark.parametrize("src,offset", [(F16, 0), (BF16, 0), (BF16, 1), (F32, 0)])
+def test_engine_attention_appends_and_attends(lia, O, kv, src, offset):
+    """Engine.attention over rows of every type and alignment (appended by the attention launch where
+    the pool's type and 16-byte alignment allow, else before it), two layers on one staged plan, then
+    a second stage of another shape: pools bit for bit and outputs against the float64 oracle."""
+    eng = lia.Engine(16, 2, 128, pool_tokens=2048, layers=2, page_size=32, kv_dtype=kv, q_dtype=F32,
+                     out_dtype=F32, prefill_batch=256)
+    eng.configure_paging(4, 1024)
+    rng = np.random.default_rng(17)
+    tables = [[int(x) for x in t] for t in np.split(rng.permutation(64), [16, 40])]
+    pools = []
+    for layer in range(2):
+        kv_np = [O.from_f32(rng.standard_normal((2048, 2, 128)).astype(np.float32), kv) if kv != FP8
+                 else rng.integers(0, 120, (2048, 2, 128)).astype(np.uint8) for _ in "kv"]
+        for dst, a in zip((eng.k[layer], eng.v[layer]), kv_np):
+            (dst if kv == FP8 else dst.view(torch.int16)).copy_(G.to_dev(a.view(np.int16) if kv != FP8 else a).view(2048, 2, 128))
+        if kv == FP8:
+            eng.k_scales[layer].fill_(0.01)
+            eng.v_scales[layer].fill_(0.02)
+        pools.append([a.reshape(-1).copy() for a in kv_np])
+    tdt = {F32: torch.float32, F16: torch.float16, BF16: torch.bfloat16}[src]
+    scales = [np.full(64 * 2, x, np.float32) if kv == FP8 else None for x in (0.01, 0.02)]
+    for rows in ([(1, p, 0) for p in range(100, 103)] + [(1, 500, 1)],
+                 [(1, p, 2) for p in range(0, 70)] + [(1, 501, 1)]):
+        packed = eng.stage(rows, tables, outputs=[0])
+        n = len(rows)
+        for layer in range(2):
+            q = rng.standard_normal((n, 16, 128)).astype(np.float32)
+            new = [rng.standard_normal((n, 256)).astype(np.float32) for _ in "kv"]
+            new = new if src == F32 else [O.from_f32(x, src) for x in new]
+
+            def dev(a):
+                t = G.to_dev(np.concatenate([np.zeros(offset, a.dtype), a.reshape(-1)]))
+                return (t if src == F32 else t.view(tdt))[offset:].view(n, 2, 128)
+
+            out = eng.attention(layer, G.to_dev(q), dev(new[0]), dev(new[1]))
+            torch.cuda.synchronize()
+            kc, vc = pools[layer]
+            O.kv_append(O.KVLayout(2, 128, 32, 64, kv), packed["positions"], packed["sequences"],
+                        packed["flat"], packed["stride"], new[0], new[1], kc, vc, src_dtype=src,
+                        k_scales=scales[0], v_scales=scales[1])
+            got = [x if kv == FP8 else x.view(torch.int16) for x in (eng.k[layer], eng.v[layer])]
+            store = np.uint8 if kv == FP8 else np.uint16
+            assert np.array_equal(got[0].cpu().numpy().view(store).reshape(-1), kc)
+            assert np.array_equal(got[1].cpu().numpy().view(store).reshape(-1), vc)
+            ref = O.attention_f64(O.geom(16, 2, 128, 32, packed["stride"], kv), packed["positions"],
+                                  packed["sequences"], packed["flat"], q, kc, vc, *scales)
+            err = np.abs(out.cpu().numpy() - ref)
+            assert err.max() < (5e-2 if kv == FP8 else 2e-2) and err.mean() < (5e-3 if kv == FP8 else 2e-3)
