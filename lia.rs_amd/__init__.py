@@ -290,7 +290,15 @@ def pack_rows(limits, rows, tables, outputs=()):
     first failing check."""
     rows = list(rows)
     n = len(rows)
-    row_arr = (PagedRow * max(n, 1))(*[PagedRow(*r) for r in rows])
+    try:
+        row_arr = np.array(rows) if n else np.zeros((1, 3), np.uint32)
+    except ValueError:  # rows of different lengths
+        row_arr = np.zeros(0)
+    if row_arr.ndim == 2 and row_arr.shape[1] == 3 and row_arr.dtype.kind in "iu":
+        row_arr = np.ascontiguousarray(row_arr.astype(np.uint32))
+        row_ptr = row_arr.ctypes.data_as(C.POINTER(PagedRow))
+    else:  # other rows: converted (or refused) one by one
+        row_arr = row_ptr = (PagedRow * n)(*[PagedRow(*r) for r in rows])
     lens = np.ascontiguousarray([len(t) for t in tables] or [0], dtype=np.uint32)
     data = np.ascontiguousarray(
         np.concatenate([np.asarray(t, dtype=np.uint32) for t in tables])
@@ -305,15 +313,14 @@ def pack_rows(limits, rows, tables, outputs=()):
     cu = np.zeros(cap + 1, np.uint32)
     slots = np.zeros(cap, np.uint32)
     info = PackInfo()
-    st = lib().lia_pack_rows(C.byref(limits), row_arr, n, data.ctypes.data, lens.ctypes.data,
+    st = lib().lia_pack_rows(C.byref(limits), row_ptr, n, data.ctypes.data, lens.ctypes.data,
                              len(tables), outs.ctypes.data, len(outputs), positions.ctypes.data,
                              sequences.ctypes.data, flat.ctypes.data, C.addressof(groups),
                              cu.ctypes.data, slots.ctypes.data, C.byref(info))
     _check(st, "pack_rows")
     g = info.n_groups
     return dict(positions=positions[:n], sequences=sequences[:n], flat=flat,
-                groups=np.array([[groups[i].start, groups[i].count, groups[i].maximum]
-                                 for i in range(g)], dtype=np.uint32).reshape(g, 3),
+                groups=np.frombuffer(groups, np.uint32).reshape(-1, 3)[:g].copy(),
                 cu_seqlens=cu[:g + 1].copy(), slot_mapping=slots[:n], stride=info.stride,
                 maximum=info.maximum, decoding=bool(info.decoding), span=info.span,
                 parts=info.parts)
@@ -897,15 +904,21 @@ class Engine:
         self.config = AttentionConfig(self.hq, self.hkv, self.d, self.page_size, self.pool_pages,
                                       stride, self.q_dtype, self.kv_dtype, self.out_dtype,
                                       self.scale, maximum_sequences, rows, context)
+        # The step's metadata lies in one device buffer with a pinned image of it, so stage() uploads
+        # it in one copy (five copies of pageable arrays took 80 us of a step).
+        sizes = dict(positions=rows, sequences=rows, slot_mapping=rows, cu_seqlens=rows + 1,
+                     pages=maximum_sequences * stride)
+        starts = np.cumsum([0] + [-(-n // 64) * 64 for n in sizes.values()])  # 256-byte aligned
+        self._meta = torch.zeros(int(starts[-1]), dtype=torch.int32, device=dev)
+        self._meta_host = torch.zeros(int(starts[-1]), dtype=torch.int32, pin_memory=True)
+        image = self._meta_host.numpy()
+        spans = {k: slice(int(b), int(b) + n) for (k, n), b in zip(sizes.items(), starts)}
+        self._meta_image = {k: image[x] for k, x in spans.items()}
         self.paging = dict(
             stride=stride,
-            positions=torch.zeros(rows, dtype=torch.int32, device=dev),
-            sequences=torch.zeros(rows, dtype=torch.int32, device=dev),
-            slot_mapping=torch.zeros(rows, dtype=torch.int32, device=dev),
-            pages=torch.zeros(maximum_sequences * stride, dtype=torch.int32, device=dev),
-            cu_seqlens=torch.zeros(rows + 1, dtype=torch.int32, device=dev),
+            **{k: self._meta[x] for k, x in spans.items()},
             workspace=torch.zeros(workspace_bytes(self.config), dtype=torch.uint8, device=dev),
-            n_seqs=0, n_rows=0)
+            n_seqs=0, n_rows=0, refused=None)
         torch.cuda.synchronize()
 
     def stage(self, rows, tables, outputs=()):
@@ -918,16 +931,21 @@ class Engine:
         w = self.paging
         n = len(packed["positions"])
         ng = len(packed["cu_seqlens"]) - 1
-        as_i32 = lambda a: torch.from_numpy(a.view(np.int32))
-        w["positions"][:n].copy_(as_i32(packed["positions"]))
-        w["sequences"][:n].copy_(as_i32(packed["sequences"]))
-        w["slot_mapping"][:n].copy_(as_i32(packed["slot_mapping"]))
-        w["pages"].copy_(as_i32(packed["flat"]))
-        w["cu_seqlens"][:ng + 1].copy_(as_i32(packed["cu_seqlens"]))
+        image = self._meta_image  # free again: every stage ends with its stream synchronised
+        for key, value in (("positions", packed["positions"]), ("sequences", packed["sequences"]),
+                           ("slot_mapping", packed["slot_mapping"]), ("pages", packed["flat"]),
+                           ("cu_seqlens", packed["cu_seqlens"])):
+            image[key][:len(value)] = value.view(np.int32)
+        self._meta.copy_(self._meta_host, non_blocking=True)
         w["n_seqs"], w["n_rows"] = ng, n
-        # the step's work list, the same for every layer
-        attention_plan(self.config, ng, n, w["cu_seqlens"], w["positions"], w["sequences"],
-                       w["workspace"], w["pages"])
+        # the step's work list, the same for every layer; a geometry the kernels refuse is attention()'s
+        # to report
+        w["refused"] = None
+        try:
+            attention_plan(self.config, ng, n, w["cu_seqlens"], w["positions"], w["sequences"],
+                           w["workspace"], w["pages"])
+        except LiaError as e:
+            w["refused"] = e
         torch.cuda.current_stream().synchronize()
         return packed
 
@@ -941,6 +959,8 @@ class Engine:
         n = w["n_rows"]
         if q.shape[0] != n or k.shape[0] != n:
             raise LiaError(-20, "attention: row count differs from the staged batch")
+        if w["refused"] is not None:
+            raise w["refused"]
         if out is None:
             odt = torch.float32 if self.out_dtype == F32 else torch.bfloat16
             out = torch.empty((n, self.hq, self.d), dtype=odt, device=q.device)
