@@ -271,21 +271,29 @@ __global__ __launch_bounds__(256) void quantize8_kernel(uint32_t n_waves, uint32
 // inv_i = f32(1 / f32(base^(2i/head_dim))), the rounded steps of coefficients
 // (src/gpu/kernels/llama_position.rs:36-47).  pow, cos and sin are evaluated in double and
 // rounded once to f32.
+//
+// One thread per column and ROWS rows 256 / half apart: the column's inverse frequency once, and
+// one argument reduction for the sine and the cosine.  Bound by the double-precision functions: 4,096
+// rows of 128 took 4.73 us with a pow, a cos and a sin per entry, 3.48 us so.
+template <uint32_t ROWS>
 __global__ __launch_bounds__(256) void rope_coefficients_kernel(uint32_t rows, uint32_t head_dim,
                                                                 float base,
                                                                 const uint32_t *positions,
                                                                 float *out) {
-    const uint32_t half = head_dim / 2;
-    const uint32_t i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= rows * half) return;
-    const float e = 2.0f * (float)(i % half) / (float)head_dim;
+    const uint32_t half = head_dim / 2, column = threadIdx.x % half, step = 256 / half;
+    const uint32_t r0 = blockIdx.x * step * ROWS + threadIdx.x / half;
+    const float e = 2.0f * (float)column / (float)head_dim;
     const float p = (float)pow((double)base, (double)e);
     const float inv = 1.0f / p;
-    const float angle = (float)positions[i / half] * inv;
-    float2 cs;
-    cs.x = (float)cos((double)angle);
-    cs.y = (float)sin((double)angle);
-    ((float2 *)out)[i] = cs;
+#pragma unroll
+    for (uint32_t k = 0; k < ROWS; k++) {
+        const uint32_t r = r0 + k * step;
+        if (r >= rows) return;
+        const float angle = (float)positions[r] * inv;
+        double c, s;
+        sincos((double)angle, &s, &c);
+        ((float2 *)out)[(size_t)r * half + column] = make_float2((float)c, (float)s);
+    }
 }
 
 template <int KVT>
@@ -402,10 +410,18 @@ extern "C" int lia_rope_coefficients(uint32_t rows, uint32_t head_dim, float bas
     if (head_dim != 64 && head_dim != 128) return LIA_E_UNSUPPORTED;
     if (((uintptr_t)coefficients & 7) != 0) return LIA_E_ALIGN;
     if (rows == 0) return LIA_OK;
-    const uint32_t n = rows * (head_dim / 2);
-    const hipError_t e = launch<rope_coefficients_kernel>(dim3((n + 255) / 256), dim3(256), 0,
-                                                          (hipStream_t)stream, rows, head_dim, base,
-                                                          positions, coefficients);
+    // More rows a thread once that leaves every CU two workgroups: one, two and four rows a thread
+    // measured 2.94, 2.81 and 3.48 us at 512 groups (2,048 rows of 128), 4.27, 3.48 and 3.65 at
+    // 1,024, 6.56, 5.12 and 4.56 at 2,048.
+    const uint32_t step = 256 / (head_dim / 2);
+    const uint32_t groups = (uint32_t)(((uint64_t)rows + step - 1) / step);
+    const uint32_t per = groups >= 2048 ? 4 : groups >= 512 ? 2 : 1;
+    const dim3 grid((groups + per - 1) / per), block(256);
+    hipStream_t s = (hipStream_t)stream;
+    hipError_t e;
+    if (per == 4) e = launch<rope_coefficients_kernel<4>>(grid, block, 0, s, rows, head_dim, base, positions, coefficients);
+    else if (per == 2) e = launch<rope_coefficients_kernel<2>>(grid, block, 0, s, rows, head_dim, base, positions, coefficients);
+    else e = launch<rope_coefficients_kernel<1>>(grid, block, 0, s, rows, head_dim, base, positions, coefficients);
     return e == hipSuccess ? LIA_OK : LIA_E_HIP;
 }
 

@@ -24,6 +24,19 @@ def test_coefficients_bit_exact(lia, O, d):
     assert np.array_equal(got.view(np.uint32), ref.view(np.uint32))
 
 
+@pytest.mark.parametrize("d,rows", [(64, 4095), (64, 4096), (64, 16385), (128, 2044), (128, 2045), (128, 8188),
+                                    (128, 8189), (128, 8195)])
+def test_coefficients_of_many_rows(lia, O, d, rows):
+    """Row counts at the edges of one, two and four rows a thread, against the oracle and without a
+    write past the table."""
+    positions = np.random.default_rng(rows).integers(0, 131072, rows).astype(np.uint32)
+    ref = O.rope_coefficients(positions, d).reshape(-1)
+    out = torch.full((ref.size + 512,), 7.0, device="cuda")
+    lia.rope_coefficients(G.u32_dev(positions), d, out)
+    got = out.cpu().numpy()
+    assert np.array_equal(got[:ref.size].view(np.uint32), ref.view(np.uint32)) and np.all(got[ref.size:] == 7.0)
+
+
 def _run(lia, O, hq, hkv, d, kv, qdt, page, use_slots, seed):
     rng = np.random.default_rng(seed)
     stride, rows = 64, 9
