@@ -22,6 +22,11 @@ namespace lia {
 // attention output is left untouched.
 constexpr uint32_t kPackHash = 8192;  // LDS slot hash (open addressing, load <= 1/2 per pass)
 constexpr uint32_t kPackPass = kPackHash / 2;
+constexpr uint32_t kPackPages = 4096; // pages of a batch's runs of rows (load <= 1/2)
+template <uint32_t N>
+struct Count {
+    static constexpr uint32_t value = N;
+};
 
 // Home bucket of a slot: the 16 slots of an aligned 16-slot group (the consecutive rows of a
 // page) take the 16 buckets of one bucket group, chosen by a multiplicative hash of the group
@@ -62,7 +67,8 @@ __device__ void pack_rows_block(uint32_t n_seqs, const uint32_t *seq_slots, cons
                                 uint32_t *sequences, uint32_t *slot_mapping, uint32_t *status,
                                 uint32_t *verdict) {
     __shared__ uint32_t scan[1024], s_slot[1024], s_c0[1024];
-    __shared__ uint32_t h_key[kPackHash], h_row[kPackHash];
+    __shared__ __attribute__((aligned(16))) uint32_t h_key[kPackHash];
+    __shared__ uint32_t h_row[kPackHash];
     __shared__ uint32_t w_a[16], w_b[16];
     // error: (row << 4) | code of the failing row with the lowest index, so the status is the
     // first failure in row order whatever the thread timing (codes are below 16)
@@ -70,16 +76,9 @@ __device__ void pack_rows_block(uint32_t n_seqs, const uint32_t *seq_slots, cons
     __shared__ uint32_t carry, error, dup;
     const uint32_t t = threadIdx.x;
     if (t == 0) { carry = 0; error = 0xFFFFFFFFu; dup = 0; }
-    for (uint32_t i = t; i < kPackHash; i += 1024) { h_key[i] = kNone; h_row[i] = kNone; }
+    static_assert(kPackPages == 4 * 1024 && kPackPages <= kPackHash, "one quad of the page table per thread");
+    ((u32x4 *)h_key)[t] = u32x4{kNone, kNone, kNone, kNone};
     const uint32_t P = 1u << page_shift;
-    auto upper = [&](const uint32_t *arr, uint32_t n, uint32_t v) { // smallest b with arr[b] > v
-        uint32_t a = 0, e = n;
-        while (a < e) {
-            const uint32_t mid = (a + e) >> 1;
-            if (arr[mid] > v) e = mid; else a = mid + 1;
-        }
-        return a;
-    };
     for (uint32_t base = 0; base < n_seqs; base += 1024) {
         const uint32_t b = base + t;
         const uint32_t n = b < n_seqs ? q_lens[b] : 0;
@@ -114,11 +113,23 @@ __device__ void pack_rows_block(uint32_t n_seqs, const uint32_t *seq_slots, cons
         reject((uint32_t)(-LIA_E_ROWS));
         return;
     }
-    // Duplicate slots: slots are hashed keeping the lowest row per slot; a row whose slot has a
-    // lower row fails.  Up to kPackPass rows take one pass, inserted while the rows are filled;
-    // larger batches take one pass per hash class of slots (slot % passes), reading the slots
-    // back.
+    // Duplicate slots.  Two rows can only share a slot if two runs of rows - a run: a sequence's rows
+    // in one logical page - lie in one physical page, so each run's first row enters its page in a
+    // small LDS table, and only when a page is entered twice are the slots themselves compared: hashed
+    // keeping the lowest row per slot, a row whose slot has a lower row fails, in one pass per hash
+    // class of slots (slot % passes) of up to kPackPass rows each.  (Hashing every row's slot took
+    // 9.4 us for 4,358 rows beside the 3.2 of the launches, and 6 for 3,589; the runs take 5.2 and 4.9.)
     const uint32_t passes = (total + kPackPass - 1) / kPackPass;
+    const bool by_page = n_seqs <= 1024 && (total >> page_shift) + n_seqs <= kPackPages / 2;
+    auto enter = [&](uint32_t page) {
+        uint32_t h = (page * 2654435761u) >> 20; // 12 bits
+        for (;;) { // the table is at most half full
+            const uint32_t k = atomicCAS(&h_key[h], kNone, page);
+            if (k == page) dup = 1;
+            if (k == page || k == kNone) return;
+            h = (h + 1) & (kPackPages - 1);
+        }
+    };
     auto insert = [&](uint32_t s, uint32_t r) {
         uint32_t h = slot_hash(s), probes = 0;
         for (; probes < kPackHash; probes++) {
@@ -158,63 +169,49 @@ __device__ void pack_rows_block(uint32_t n_seqs, const uint32_t *seq_slots, cons
     auto page_of = [&](uint32_t pos, uint32_t slot) {
         return pos < context ? pages[(size_t)slot * stride + (pos >> page_shift)] : kNone;
     };
-    if (n_seqs <= 1024 && passes <= 1) {
-        // Rows in parallel (at most 4 per thread, slots kept in registers): row r belongs to
-        // the first sequence whose inclusive prefix sum exceeds r.  The rows' page loads are
-        // issued together with the table check's.
-        constexpr uint32_t RPT = kPackPass / 1024;
-        uint32_t mine[RPT], pos[RPT], sl[RPT], pg[RPT];
-        auto rows = [&] {
-            uint32_t rr[RPT], seq[RPT];
+    if (n_seqs <= 1024) {
+        // Rows in parallel, K a thread and batch: row r belongs to the first sequence whose
+        // inclusive prefix sum exceeds r.  The page loads of a batch are issued together.
+        auto rows = [&](auto k_rows, uint32_t base) {
+            constexpr uint32_t K = decltype(k_rows)::value;
+            uint32_t rr[K], seq[K], first[K], pg[K];
 #pragma unroll
-            for (uint32_t k = 0; k < RPT; k++) rr[k] = min(t + k * 1024, total ? total - 1 : 0u);
-            upper_many<RPT>(scan, n_seqs, rr, seq);
+            for (uint32_t k = 0; k < K; k++) rr[k] = min(base + t + k * 1024, total ? total - 1 : 0u);
+            upper_many<K>(scan, n_seqs, rr, seq);
 #pragma unroll
-            for (uint32_t k = 0; k < RPT; k++) {
-                const uint32_t r = t + k * 1024, a = seq[k];
-                pos[k] = s_c0[a] + r - (a ? scan[a - 1] : 0u);
-                sl[k] = s_slot[a];
-                pg[k] = r < total ? page_of(pos[k], sl[k]) : kNone;
+            for (uint32_t k = 0; k < K; k++) {
+                first[k] = seq[k] ? scan[seq[k] - 1] : 0u;
+                pg[k] = page_of(s_c0[seq[k]] + rr[k] - first[k], s_slot[seq[k]]);
+            }
+#pragma unroll
+            for (uint32_t k = 0; k < K; k++) {
+                if (base + t + k * 1024 >= total) continue;
+                const uint32_t pos = s_c0[seq[k]] + rr[k] - first[k];
+                const uint32_t slot = finish(rr[k], pos, s_slot[seq[k]], pg[k]);
+                if (by_page && slot != kNone && (rr[k] == first[k] || (pos & (P - 1)) == 0)) enter(slot >> page_shift);
             }
         };
-        rows();
-#pragma unroll
-        for (uint32_t k = 0; k < RPT; k++) {
-            const uint32_t r = t + k * 1024;
-            mine[k] = kNone;
-            if (r < total) {
-                mine[k] = finish(r, pos[k], sl[k], pg[k]);
-                if (mine[k] != kNone) insert(mine[k], r);
-            }
-        }
-        lds_barrier(); // the hash (LDS); the rows' global stores need not have landed
-        if (dup) { // uniform; with no slot inserted twice no row can fail
-#pragma unroll
-            for (uint32_t k = 0; k < RPT; k++)
-                if (mine[k] != kNone) lookup(mine[k], t + k * 1024);
+        if (total <= 1024) {
+            if (total) rows(Count<1>{}, 0); // (without rows no sequence holds row 0)
+        } else {
+            for (uint32_t base = 0; base < total; base += kPackPass) rows(Count<kPackPass / 1024>{}, base);
         }
     } else {
-        if (n_seqs <= 1024) {
-            for (uint32_t r = t; r < total; r += 1024) {
-                const uint32_t a = upper(scan, n_seqs, r);
-                const uint32_t p = s_c0[a] + r - (a ? scan[a - 1] : 0u);
-                finish(r, p, s_slot[a], page_of(p, s_slot[a]));
-            }
-        } else {
-            // more sequences than the LDS copies hold: walk sequences, threads stride over each
-            // sequence's rows
-            for (uint32_t b = 0; b < n_seqs; b++) {
-                const uint32_t start = cu[b], n = q_lens[b], slot = seq_slots[b], c0 = cached[b];
-                for (uint32_t i = t; i < n; i += 1024) finish(start + i, c0 + i, slot, page_of(c0 + i, slot));
-            }
+        // more sequences than the LDS copies hold: walk sequences, threads stride over each
+        // sequence's rows
+        for (uint32_t b = 0; b < n_seqs; b++) {
+            const uint32_t start = cu[b], n = q_lens[b], slot = seq_slots[b], c0 = cached[b];
+            for (uint32_t i = t; i < n; i += 1024) finish(start + i, c0 + i, slot, page_of(c0 + i, slot));
         }
+    }
+    lds_barrier(); // the pages (LDS); the rows' global stores need not have landed
+    if (!by_page || dup) { // uniform
         __threadfence_block(); // this workgroup's slot_mapping writes, read back below
         __syncthreads();
+        if (t == 0) dup = 0;
         for (uint32_t pass = 0; pass < passes; pass++) {
-            if (pass) {
-                for (uint32_t i = t; i < kPackHash; i += 1024) { h_key[i] = kNone; h_row[i] = kNone; }
-                __syncthreads();
-            }
+            for (uint32_t i = t; i < kPackHash; i += 1024) { h_key[i] = kNone; h_row[i] = kNone; }
+            __syncthreads();
             for (uint32_t r = t; r < total; r += 1024) {
                 const uint32_t s = slot_mapping[r];
                 if (s != kNone && s % passes == pass) insert(s, r);

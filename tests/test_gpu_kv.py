@@ -353,3 +353,61 @@ def test_engine_attention_appends_and_attends(lia, O, kv, src, offset):
                                   packed["sequences"], packed["flat"], q, kc, vc, *scales)
             err = np.abs(out.cpu().numpy() - ref)
             assert err.max() < (5e-2 if kv == FP8 else 2e-2) and err.mean() < (5e-3 if kv == FP8 else 2e-3)
+
+
+def _pack_both(lia, q_len, cached, tables, P, pool):
+    """The device's packing (both entry points' checks) and the host's, of one batch: their metadata,
+    or their failure codes."""
+    n, rows = len(q_len), int(sum(q_len))
+    stride = max(len(t) for t in tables)
+    context = stride * P
+    flat = np.full(n * stride, 0xFFFFFFFF, np.uint32)
+    for i, t in enumerate(tables):
+        flat[i * stride:i * stride + len(t)] = t
+    out = [torch.full((max(m, 1),), -7, dtype=torch.int32, device="cuda") for m in (n + 1, rows, rows, rows, 1)]
+    lia.pack_device(G.u32_dev(np.arange(n)), G.u32_dev(q_len), G.u32_dev(cached), G.u32_dev(flat), stride, P, pool,
+                    context, max(rows, 1), *out)
+    torch.cuda.synchronize()
+    status = int(out[4].item())
+    if rows == 0:
+        return status, None
+    host_rows = [(0, int(c) + i, s) for s, (q, c) in enumerate(zip(q_len, cached)) for i in range(int(q))]
+    try:
+        packed = lia.pack_rows(lia.PagingLimits(n, context, P, pool, 1, rows), host_rows, [list(map(int, t)) for t in tables])
+    except lia.LiaError as e:
+        return status, -e.status
+    got = [o.cpu().numpy().view(np.uint32) for o in out[:4]]
+    assert status == 0
+    assert np.array_equal(got[1], packed["positions"]) and np.array_equal(got[2], packed["sequences"])
+    assert np.array_equal(got[3], packed["slot_mapping"])
+    return 0, 0
+
+
+@pytest.mark.parametrize("P,q_len", [(16, [5000, 3]), (16, [1] * 700), (16, [0, 1023, 0, 1, 1]), (64, [4097]),
+                                     (16, [4090, 1, 1, 1, 1, 1, 1]), (1, [3000, 17]), (2, [5000]), (16, [0, 0])])
+def test_pack_device_row_counts(lia, P, q_len):
+    """Batches about the packing's limits (1,024 rows a pass, 4,096 a batch, the table of the runs'
+    pages, pages of one and two tokens, no rows at all) equal the host's."""
+    rng = np.random.default_rng(sum(q_len) + P)
+    cached = rng.integers(0, 50, len(q_len))
+    need = [-(-(int(q) + int(c)) // P) for q, c in zip(q_len, cached)]
+    pool = max(sum(need), 1) + 3
+    perm = rng.permutation(pool)
+    tables = [x for x in np.split(perm[:sum(need)], np.cumsum(need)[:-1])]
+    tables = [t if len(t) else perm[:1] for t in tables]
+    status, want = _pack_both(lia, q_len, cached, tables, P, pool)
+    assert status == (want or 0)
+
+
+@pytest.mark.parametrize("big", [False, True])
+@pytest.mark.parametrize("other,want", [(6, 0), (5, 11), (3, 11)])
+def test_pack_device_rows_sharing_a_page(lia, big, other, want):
+    """Two sequences whose new rows lie in one physical page: accepted while their slots differ (rows
+    3 to 5 of one and 6 on of the other), rejected at the first slot written twice; alone and behind
+    4,500 rows."""
+    P, pool = 16, 400
+    q_len, cached, tables = [3, 2], [3, other], [[7], [7]]
+    if big:
+        q_len, cached, tables = [4500] + q_len, [0] + cached, [list(range(100, 100 + -(-4500 // P)))] + tables
+    status, host = _pack_both(lia, q_len, cached, tables, P, pool)
+    assert status == host == want
