@@ -62,7 +62,7 @@ constexpr uint32_t kPrePages = 4;
 struct WorkDesc {
     uint32_t unit;            // first unit of the range
     uint32_t lo, hi;          // block range [lo, hi)
-    uint32_t flags;           // bit 0: pre[] valid; bits 8-31: range index (record base)
+    uint32_t flags;           // bit 0: pre[] valid; bits 8-31: range index (record base, signed)
     UnitDesc first;           // units[unit]
     uint4 pre;                // pages of logical pages (32 * (lo - first.block_start)) / P + 0..3
 };
@@ -154,6 +154,7 @@ __device__ __forceinline__ uint32_t div_by(uint64_t a, uint64_t b, double inv) {
 
 constexpr uint32_t kPlanSeqs = 1024; // sequences the plan keeps in LDS (one per thread)
 constexpr uint32_t kPlanThreads = 1024;
+constexpr uint32_t kQueueGroups = 2048; // pieces per KV head a queue holds at most
 // Workgroups of plan_lds_kernel: each computes the per-sequence extents and then writes an
 // interleaved share of the descriptors (one workgroup issued them all at 16 waves on one CU).
 constexpr uint32_t kPlanGroups = 8;
@@ -206,10 +207,22 @@ constexpr uint32_t kLagWide = 56, kLagDecode = 0;
 //    bits and 9/16 in f32 (written and read at 5 TB/s).  4 chunks of 512 rows, 32 query / 8 KV
 //    heads, from empty caches 52.6 -> 37.4 us, on 4,000 keys 181.8 -> 159.4; 8 of 256 rows on
 //    4,000 keys 201 -> 156; two heads and 256 units on 4,000 keys stay split (97 us; 122 unsplit).
+//
+// A queue (prefill, more units than resident workgroups): one workgroup per unit, units longer than
+// half an even share of the CUs cut into equal pieces, launched longest first, so the hardware's
+// dispatch evens them out: a freed CU takes the next, shorter one.  Even ranges end together only in
+// blocks, not in time (a range's blocks differ in masking, loads and neighbours), and leave about two
+// records a workgroup.  Taken when the end it leaves uneven (the longest piece of the last round, in
+// the eighths of a block above) and the records of its cut units cost less than those records: four
+// chunks of about 2,048 rows from empty caches, 32 query / 8 KV heads, 293 -> 268 us; six of about
+// 1,000 rows on 700 keys 194 -> 184; ten of 600 rows, 16 / 2 heads, 68 -> 59; four FP8 chunks of 33 to
+// 2,048 rows on 0 to 12,000 keys 235 -> 227.  Long units of few heads stay ranges (eight chunks of 700
+// rows on 1,500 keys, two heads, 114 us).
 struct PlanRule {
     uint32_t unit_cost;  // virtual blocks charged to each unit
     uint32_t round_wg, lag, xcd;
     uint32_t small_cost, span_shift;
+    uint32_t n_more;     // work descriptors past n_wg (0: no queue)
     uint32_t rec;        // prefill: a record's cost (16ths of an eighth of a block); decode: 0
 };
 
@@ -218,7 +231,7 @@ struct RawSeqs {
     uint32_t n_rows;
 };
 
-template <bool RAW>
+template <bool RAW, bool QUEUE>
 __device__ __forceinline__ void plan_lds(uint32_t n_seqs, const uint32_t *cu, const uint32_t *positions,
                                          const uint32_t *sequences, const RawSeqs &raw,
                                          const uint32_t *pages, uint32_t stride, uint32_t page_shift,
@@ -233,6 +246,7 @@ __device__ __forceinline__ void plan_lds(uint32_t n_seqs, const uint32_t *cu, co
     __shared__ uint32_t w_s[4][kPlanThreads / 64], w_long[kPlanThreads / 64];
     __shared__ uint32_t carry_units, carry_blocks, carry_rows, raw_bad;
     __shared__ uint32_t s_rlo[kPlanThreads + 1];
+    __shared__ uint32_t s_hist[QUEUE ? 256 : 1], s_item[QUEUE ? kQueueGroups : 1], s_q[3];
     // Threads exchange only LDS data (nothing written to global memory is read back), so the
     // barriers need not wait for the descriptor stores in flight.
     constexpr uint32_t T = kPlanThreads;
@@ -320,6 +334,69 @@ __device__ __forceinline__ void plan_lds(uint32_t n_seqs, const uint32_t *cu, co
         aligned = U && U <= n_wg && one * N <= share + records * N;
         if (aligned) N = U;
     }
+    // last index a of arr[0 .. n) (ascending, arr[0] <= v) with arr[a] <= v.  On sequences: empty
+    // ones share their offset with the next, so this is the sequence that owns v.
+    auto last_le = [&](const uint32_t *arr, uint32_t n, uint32_t v) {
+        uint32_t a = 0, e = n;
+#pragma unroll 1
+        while (a + 1 < e) {
+            const uint32_t mid = (a + e) >> 1;
+            if (arr[mid] <= v) a = mid; else e = mid;
+        }
+        return a;
+    };
+    // The queue (PlanRule): column block g of the batch (of one KV head), cut into pieces of at most
+    // `cut` blocks; pieces are ordered by length class, longest first.
+    bool queue = false;
+    const uint32_t cut = (uint32_t)((TC + 2 * rule.round_wg - 1) / max(1u, 2 * rule.round_wg));
+    const uint32_t class_shift = cut > 255 ? 24 - __builtin_clz(cut) : 0;
+    struct Cut { uint32_t b, cb, len, pieces, cls; };
+    auto cut_of = [&](uint32_t g) {
+        Cut c;
+        c.b = last_le(s_u0, n_seqs, g * hkv);
+        c.cb = g - s_u0[c.b] / hkv;
+        c.len = unit_blocks(s_p0[c.b], min((c.cb + 1) * rpc, s_nr[c.b]));
+        c.pieces = (c.len + cut - 1) / cut;
+        c.cls = 255 - min(((c.len + c.pieces - 1) / c.pieces) >> class_shift, 255u);
+        return c;
+    };
+    if (QUEUE && U > n_wg && TC < (uint64_t)rule.small_cost) { // uniform
+        if (t < 256) s_hist[t] = 0;
+        if (t < 3) s_q[t] = 0;
+        lds_barrier();
+        for (uint32_t g = t; g < U / hkv; g += T) {
+            const Cut c = cut_of(g);
+            atomicAdd(&s_hist[c.cls], c.pieces);
+            if (c.pieces > 1) atomicAdd(&s_q[0], c.pieces);
+        }
+        lds_barrier();
+        if (t < 64) { // exclusive sums over the classes; the class of the last round's longest piece
+            uint32_t n[4], sum = 0;
+#pragma unroll
+            for (int i = 0; i < 4; i++) { n[i] = s_hist[4 * t + i]; sum += n[i]; }
+            uint32_t at = sum;
+#pragma unroll
+            for (int off = 1; off < 64; off <<= 1) {
+                const uint32_t x = __shfl_up(at, off);
+                if (lane >= (uint32_t)off) at += x;
+            }
+            const uint32_t all = __shfl(at, 63), round = 2 * rule.round_wg / hkv;
+            const uint32_t mark = all > round ? all - round : 0;
+            at -= sum;
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                s_hist[4 * t + i] = at;
+                if (at <= mark && mark < at + n[i]) s_q[2] = 4 * t + i;
+                at += n[i];
+            }
+            if (t == 0) s_q[1] = all;
+        }
+        lds_barrier();
+        const uint32_t all = s_q[1], items = all * hkv, tail = (256 - s_q[2]) << class_shift;
+        queue = all <= kQueueGroups && items > n_wg && items <= n_wg + rule.n_more &&
+                8 * tail + (s_q[0] * hkv * rule.rec >> 4) <= (2 * n_wg * rule.rec >> 4);
+        if (queue) N = items;
+    }
     if (t == 0) {
         s_u0[n_seqs] = carry_units;
         s_b0[n_seqs] = carry_blocks;
@@ -359,7 +436,7 @@ __device__ __forceinline__ void plan_lds(uint32_t n_seqs, const uint32_t *cu, co
     // of 256 spans TC * w / F(N) >= TC * (256 - lag) / F(N), so with that at least 1 each start
     // lies at least one block after the previous one.  A range empty in blocks inside a unit
     // would be counted among the unit's records without writing one.
-    bool skew = !aligned && lag && round_wg && round_wg < N;
+    bool skew = !aligned && !queue && lag && round_wg && round_wg < N;
     uint64_t FN = N; // the weights' sum (equal weights: one each)
     if (skew) {
         const uint64_t weighted = 256ull * N - (uint64_t)lag * late_before(N);
@@ -375,17 +452,6 @@ __device__ __forceinline__ void plan_lds(uint32_t n_seqs, const uint32_t *cu, co
     }
     lds_barrier();
     auto range_lo = [&](uint32_t r) -> uint32_t { return skew ? s_rlo[r] : div_by(r * TC, FN, inv_n); };
-    // last index a of arr[0 .. n) (ascending, arr[0] <= v) with arr[a] <= v.  On sequences: empty
-    // ones share their offset with the next, so this is the sequence that owns v.
-    auto last_le = [&](const uint32_t *arr, uint32_t n, uint32_t v) {
-        uint32_t a = 0, e = n;
-#pragma unroll 1
-        while (a + 1 < e) {
-            const uint32_t mid = (a + e) >> 1;
-            if (arr[mid] <= v) a = mid; else e = mid;
-        }
-        return a;
-    };
     auto make_unit = [&](uint32_t b, uint32_t h, uint32_t cb) {
         const uint32_t p0 = s_p0[b], cblocks = (p0 + 31) / 32;
         const uint32_t rows = min(rpc, s_nr[b] - cb * rpc), kend = p0 + cb * rpc + rows;
@@ -393,6 +459,59 @@ __device__ __forceinline__ void plan_lds(uint32_t n_seqs, const uint32_t *cu, co
         return UnitDesc{blk, unit_blocks(p0, kend - p0), cblocks, s_r0[b] + cb * rpc, rows | (h << 16),
                         kend, s_trow[b], p0};
     };
+    // A work descriptor of blocks [lo, hi), the first in column block cb of KV head h of sequence b.
+    auto emit = [&](WorkDesc *to, uint32_t b, uint32_t h, uint32_t cb, uint32_t lo, uint32_t hi, uint32_t tag) {
+        WorkDesc d;
+        d.unit = s_u0[b] + h * s_ncb[b] + cb;
+        d.first = make_unit(b, h, cb);
+        d.flags = tag << 8;
+        d.lo = lo;
+        d.hi = hi;
+        // logical pages the range starts with, when it starts in the cached keys (unconditional
+        // page-table loads: an entry not needed reads a word the plan reads anyway - cu[0], or
+        // q_lens[0] of a raw plan - and is replaced by 0)
+        const uint32_t *dummy = RAW ? raw.q_lens : cu;
+        const uint32_t rel = lo - d.first.block_start;
+        const bool pre = pages && rel < d.first.cblocks;
+        const uint32_t lp = (32 * rel) >> page_shift;
+        const uint32_t lend = (d.first.kend + (1u << page_shift) - 1) >> page_shift;
+        uint32_t v[kPrePages];
+#pragma unroll
+        for (uint32_t i = 0; i < kPrePages; i++) {
+            const bool use = pre && lp + i < lend;
+            const uint32_t *src = use ? pages + (size_t)d.first.table_row * stride + lp + i : dummy;
+            v[i] = *src;
+            v[i] = use ? v[i] : 0u;
+        }
+        if (pre) d.flags |= 1;
+        d.pre = make_uint4(v[0], v[1], v[2], v[3]);
+        *to = d;
+    };
+    if (QUEUE && queue) {
+        // One workgroup orders the pieces (its LDS counters give the places), and lists each with its
+        // unit's merge descriptor.  The pieces of a unit are consecutive items, so are its records:
+        // item i of unit u is tagged i - u.
+        if (grp == 0) {
+            for (uint32_t g = t; g < U / hkv; g += T) {
+                const Cut c = cut_of(g);
+                const uint32_t at = atomicAdd(&s_hist[c.cls], c.pieces);
+                for (uint32_t k = 0; k < c.pieces; k++) s_item[at + k] = g | k << 16;
+            }
+            lds_barrier();
+            for (uint32_t i = t; i < N; i += T) {
+                const uint32_t slot = i / hkv, item = s_item[slot], first = (slot - (item >> 16)) * hkv;
+                const Cut c = cut_of(item & 0xffffu);
+                const uint32_t h = (i - first) / c.pieces, k = i - first - h * c.pieces;
+                const UnitDesc ud = make_unit(c.b, h, c.cb);
+                const uint32_t u = s_u0[c.b] + h * s_ncb[c.b] + c.cb;
+                emit(work + i, c.b, h, c.cb, ud.block_start + k * c.len / c.pieces,
+                     ud.block_start + (k + 1) * c.len / c.pieces, (i - u) & 0xffffffu);
+                if (k == 0) merge[u] = c.pieces > 1 ? MergeDesc{i, c.pieces, ud.rowbeg, ud.nrows_hk} : MergeDesc{0, 0, 0, 0};
+            }
+        }
+        for (uint32_t u = U + g0; u < max_units; u += GT) merge[u] = MergeDesc{0, 0, 0, 0};
+        return;
+    }
     // The work descriptors, 63 ranges to a wave (each lane finds its range's start, and takes the
     // next range's from the next lane), by the last waves, so that their chain (searches, table
     // loads) runs beside the units' on the others.  Each workgroup takes contiguous ranges.
@@ -439,31 +558,7 @@ __device__ __forceinline__ void plan_lds(uint32_t n_seqs, const uint32_t *cu, co
         }
         const uint32_t hi = __shfl_down(lo, 1);
         if (lane == 63 || r >= N || r0 + lane >= share) continue;
-        WorkDesc d;
-        d.unit = s_u0[b] + h * s_ncb[b] + cb;
-        d.first = make_unit(b, h, cb);
-        d.flags = r << 8;
-        d.lo = lo;
-        d.hi = hi;
-        // logical pages the range starts with, when it starts in the cached keys (unconditional
-        // page-table loads: an entry not needed reads a word the plan reads anyway - cu[0], or
-        // q_lens[0] of a raw plan - and is replaced by 0)
-        const uint32_t *dummy = RAW ? raw.q_lens : cu;
-        const uint32_t rel = lo - d.first.block_start;
-        const bool pre = pages && rel < d.first.cblocks;
-        const uint32_t lp = (32 * rel) >> page_shift;
-        const uint32_t lend = (d.first.kend + (1u << page_shift) - 1) >> page_shift;
-        uint32_t v[kPrePages];
-#pragma unroll
-        for (uint32_t i = 0; i < kPrePages; i++) {
-            const bool use = pre && lp + i < lend;
-            const uint32_t *src = use ? pages + (size_t)d.first.table_row * stride + lp + i : dummy;
-            v[i] = *src;
-            v[i] = use ? v[i] : 0u;
-        }
-        if (pre) d.flags |= 1;
-        d.pre = make_uint4(v[0], v[1], v[2], v[3]);
-        work[w] = d;
+        emit(work + w, b, h, cb, lo, hi, r);
     }
     // each unit's descriptor, and its merge descriptor from it
 #pragma unroll 1
@@ -490,12 +585,13 @@ __device__ __forceinline__ void plan_lds(uint32_t n_seqs, const uint32_t *cu, co
     }
 }
 
+template <bool QUEUE>
 __global__ __launch_bounds__(kPlanThreads) void plan_lds_kernel(
     uint32_t n_seqs, const uint32_t *cu, const uint32_t *positions, const uint32_t *sequences,
     const uint32_t *pages, uint32_t stride, uint32_t page_shift, uint32_t rpc, uint32_t hkv,
     uint32_t max_units, uint32_t n_wg, PlanRule rule, UnitDesc *units, WorkDesc *work,
     MergeDesc *merge, uint32_t *header) {
-    plan_lds<false>(n_seqs, cu, positions, sequences, RawSeqs{}, pages, stride, page_shift, rpc, hkv, max_units,
+    plan_lds<false, QUEUE>(n_seqs, cu, positions, sequences, RawSeqs{}, pages, stride, page_shift, rpc, hkv, max_units,
              n_wg, rule, blockIdx.x, gridDim.x, units, work, merge, header);
 }
 
@@ -515,14 +611,14 @@ static_assert((kFoundWords + kSetupChecks) * 4 <= 256, "the workspace header");
 // lia_pack_plan_device's first launch (1024-thread workgroups): 0 .. kPlanGroups-1 plan the step
 // from the packing's inputs, kPlanGroups packs it (its status also to the header's verdict
 // word), and the kSetupChecks after it check the block tables.
+template <bool QUEUE>
 __global__ __launch_bounds__(kPlanThreads) void pack_plan_kernel(
     uint32_t n_seqs, PackArgs pk, RawSeqs raw, uint32_t rpc, uint32_t hkv, uint32_t max_units,
     uint32_t n_wg, PlanRule rule, UnitDesc *units, WorkDesc *work, MergeDesc *merge, uint32_t *header) {
     const uint32_t bid = blockIdx.x;
     if (bid < kPlanGroups) {
-        plan_lds<true>(n_seqs, nullptr, nullptr, nullptr, raw, pk.pages, pk.stride, pk.page_shift, rpc, hkv,
-                 max_units, n_wg, rule, bid, kPlanGroups, units, work, merge,
-                 header);
+        plan_lds<true, QUEUE>(n_seqs, nullptr, nullptr, nullptr, raw, pk.pages, pk.stride, pk.page_shift, rpc, hkv,
+                 max_units, n_wg, rule, bid, kPlanGroups, units, work, merge, header);
     } else if (bid == kPlanGroups) {
         pack_rows_block(n_seqs, pk.seq_slots, pk.q_lens, pk.cached, pk.pages, pk.stride, pk.page_shift,
                         pk.pool_pages, pk.context, pk.max_rows, pk.cu, pk.positions, pk.sequences,
@@ -2275,7 +2371,11 @@ __global__ __launch_bounds__(WCfg<D>::THREADS, 2) void wide_kernel(AttnParams p)
     __shared__ __attribute__((aligned(16))) uint16_t v0[W::STAGE], v1[W::STAGE], v2[W::STAGE], v3[S4];
     uint16_t *const st_k[4] = {k0, k1, k2, k3}, *const st_v[4] = {v0, v1, v2, v3};
     const uint32_t wg = blockIdx.x;
-    const WorkDesc wd = p.work[wg];
+    const WorkDesc wd = p.work[wg]; // (read whole before the test: behind it, the load starts 0.4 us later)
+    asm volatile("" ::"s"(wd.unit), "s"(wd.lo), "s"(wd.hi), "s"(wd.flags), "s"(wd.first.block_start),
+                 "s"(wd.first.nblocks), "s"(wd.first.cblocks), "s"(wd.first.rowbeg), "s"(wd.first.nrows_hk),
+                 "s"(wd.first.kend), "s"(wd.first.table_row), "s"(wd.first.kcache));
+    if (wg >= p.n_wg && wg >= p.header[2]) return; // past the queue (or the plan has none)
     const uint32_t tid = threadIdx.x, lane = tid & 63;
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
     const uint32_t g = lane >> 4, li = lane & 15;
@@ -2363,7 +2463,7 @@ __global__ __launch_bounds__(WCfg<D>::THREADS, 2) void wide_kernel(AttnParams p)
         }
 
         const bool whole = lo == bs && seg_end == uend;
-        const uint32_t rec = (wd.flags >> 8) + u;
+        const uint32_t rec = (uint32_t)((int)wd.flags >> 8) + u; // (a queue's tag may be negative)
 #pragma unroll
         for (int nt = 0; nt < NTW; nt++) {
             const float lt = st.l[nt][0];
@@ -2973,7 +3073,7 @@ static int run_stages(int stages, const lia_attention_config *c, uint32_t n_seqs
     p.cu = cu_seqlens; p.positions = positions; p.sequences = sequences; p.pages = pages;
     p.out = out;
     p.units = (const UnitDesc *)(ws + L.units);
-    p.work = (const WorkDesc *)(ws + L.work);
+    WorkDesc *work = (WorkDesc *)(ws + L.work);
     p.merge = (const MergeDesc *)(ws + L.merge);
     p.header = (const uint32_t *)(ws + L.header);
     p.part_o = (float *)(ws + L.part_o);
@@ -2993,11 +3093,32 @@ static int run_stages(int stages, const lia_attention_config *c, uint32_t n_seqs
     p.vc_w = const_cast<void *>(vc);
     p.n_rows = n_rows;
     p.round_wg = lia_device_cus() ? lia_device_cus() : 256;
+    // The parallel plan takes any number of workgroups (its descriptor loops stride); only its
+    // weighted range starts are an LDS table of kPlanThreads.  head_dim 64 decode launches 1,536
+    // workgroups (2,048 on FP8 pools): with the serial plan_kernel behind the two packing
+    // launches a step of 4 short sequences over two layers took 30.7 us, this way 22.6.
+    const bool parallel = n_seqs <= kPlanSeqs && (NT != kWideNT || n_wg <= kPlanThreads);
+    // A prefill batch of more units than workgroups may be planned as a queue, of up to n_more work
+    // descriptors past n_wg.  A prefill plan's descriptors therefore lie at the end of the unit list,
+    // which is sized for the decode kernel's narrower units (where a configuration leaves the room;
+    // it alone decides the place, as every array's of the workspace).
+    uint32_t n_more = 0;
+    if (NT == kWideNT) {
+        const size_t hkv = c->num_kv_heads, rounds = 2 * p.round_wg;
+        const size_t bound = ((size_t)n_rows / rpc + n_seqs) * hkv;
+        const size_t most = ((size_t)c->max_rows / rpc + c->max_seqs) * hkv + rounds;
+        const size_t end = L.units + ((size_t)L.max_units + 1) * sizeof(UnitDesc);
+        const size_t at = end > most * sizeof(WorkDesc) ? (end - most * sizeof(WorkDesc)) & ~(sizeof(WorkDesc) - 1) : 0;
+        if (most >= n_wg && most <= L.max_units && at >= L.units + (most - rounds + 1) * sizeof(UnitDesc)) {
+            work = (WorkDesc *)(ws + at);
+            if (bound > n_wg && parallel && bound / hkv <= kQueueGroups) n_more = (uint32_t)(bound + rounds) - n_wg;
+        }
+    }
+    p.work = work;
     hipStream_t s = (hipStream_t)stream;
     hipError_t e = hipSuccess;
     if (stages & kPlan) {
         UnitDesc *units = (UnitDesc *)(ws + L.units);
-        WorkDesc *work = (WorkDesc *)(ws + L.work);
         MergeDesc *merge = (MergeDesc *)(ws + L.merge);
         uint32_t *header = (uint32_t *)(ws + L.header);
         // Block ranges XCD-major (each XCD a contiguous share).  Measured against launch order:
@@ -3008,23 +3129,23 @@ static int run_stages(int stages, const lia_attention_config *c, uint32_t n_seqs
         const uint32_t lag = wide ? kLagWide : kLagDecode;
         const bool rec32 = p.out_f32 || c->kv_dtype == LIA_FP8_E4M3;
         const PlanRule rule{wide ? kUnitCostWide : kUnitCostDecode, lia_device_cus(), lag, xcd,
-                            wide ? 1u << 18 : 6 * n_wg, wide ? 0u : 1u,
+                            wide ? 1u << 18 : 6 * n_wg, wide ? 0u : 1u, n_more,
                             wide ? (rec32 ? 9u : 5u) : 0u};
-        // The parallel plan takes any number of workgroups (its descriptor loops stride); only its
-        // weighted range starts are an LDS table of kPlanThreads.  head_dim 64 decode launches 1,536
-        // workgroups (2,048 on FP8 pools): with the serial plan_kernel behind the two packing
-        // launches a step of 4 short sequences over two layers took 30.7 us, this way 22.6.
-        const bool parallel = n_seqs <= kPlanSeqs && (!lag || n_wg <= kPlanThreads);
         if (pk && parallel) {
             // the packing, the plan (from the packing's inputs) and the table checks in one
             // launch, then the step's verdict
             const RawSeqs raw{pk->q_lens, pk->cached, pk->seq_slots, n_rows};
-            e = launch<pack_plan_kernel>(dim3(kPlanGroups + 1 + kSetupChecks), dim3(kPlanThreads), 0, s,
-                                         n_seqs, *pk, raw, rpc, c->num_kv_heads, L.max_units, n_wg, rule, units, work, merge, header);
+            const dim3 grid(kPlanGroups + 1 + kSetupChecks);
+            if (n_more)
+                e = launch<pack_plan_kernel<true>>(grid, dim3(kPlanThreads), 0, s, n_seqs, *pk, raw, rpc,
+                                                   c->num_kv_heads, L.max_units, n_wg, rule, units, work, merge, header);
+            else
+                e = launch<pack_plan_kernel<false>>(grid, dim3(kPlanThreads), 0, s, n_seqs, *pk, raw, rpc,
+                                                    c->num_kv_heads, L.max_units, n_wg, rule, units, work, merge, header);
             if (e == hipSuccess)
                 e = launch<setup_verdict_kernel>(dim3(1), dim3(kPlanThreads), 0, s, n_seqs, pk->max_rows,
-                                                 pk->cu, pk->slot_mapping, pk->status, header, work, n_wg,
-                                                 merge, L.max_units);
+                                                 pk->cu, pk->slot_mapping, pk->status, header, work,
+                                                 n_wg + n_more, merge, L.max_units);
         } else {
             if (pk) { // too many sequences for the one-launch form: pack first
                 const int ps = lia_pack_device(n_seqs, pk->seq_slots, pk->q_lens, pk->cached, pk->pages,
@@ -3033,10 +3154,14 @@ static int run_stages(int stages, const lia_attention_config *c, uint32_t n_seqs
                                                pk->sequences, pk->slot_mapping, pk->status, stream);
                 if (ps) return ps;
             }
-            if (parallel)
-            e = launch<plan_lds_kernel>(dim3(kPlanGroups), dim3(kPlanThreads), 0, s, n_seqs, cu_seqlens,
-                                        positions, sequences, pages, c->stride, p.page_shift, rpc,
-                                        c->num_kv_heads, L.max_units, n_wg, rule, units, work, merge, header);
+            if (n_more)
+                e = launch<plan_lds_kernel<true>>(dim3(kPlanGroups), dim3(kPlanThreads), 0, s, n_seqs, cu_seqlens,
+                                                  positions, sequences, pages, c->stride, p.page_shift, rpc,
+                                                  c->num_kv_heads, L.max_units, n_wg, rule, units, work, merge, header);
+            else if (parallel)
+                e = launch<plan_lds_kernel<false>>(dim3(kPlanGroups), dim3(kPlanThreads), 0, s, n_seqs, cu_seqlens,
+                                                   positions, sequences, pages, c->stride, p.page_shift, rpc,
+                                                   c->num_kv_heads, L.max_units, n_wg, rule, units, work, merge, header);
             else
             e = launch<plan_kernel>(dim3(1), dim3(256), 0, s, n_seqs, cu_seqlens, positions,
                                     sequences, pages, c->stride, p.page_shift, rpc, c->num_kv_heads,
@@ -3047,11 +3172,11 @@ static int run_stages(int stages, const lia_attention_config *c, uint32_t n_seqs
         if (c->head_dim == 128) {
             if (NT == 1) e = launch_partial_kv<128, 1>(c->kv_dtype, p, n_wg, s);
             else if (NT == 2) e = launch_partial_kv<128, 2>(c->kv_dtype, p, n_wg, s);
-            else e = launch_wide<128>(c->kv_dtype, p, n_wg, s);
+            else e = launch_wide<128>(c->kv_dtype, p, n_wg + n_more, s);
         } else {
             if (NT == 1) e = launch_partial_kv<64, 1>(c->kv_dtype, p, n_wg, s);
             else if (NT == 2) e = launch_partial_kv<64, 2>(c->kv_dtype, p, n_wg, s);
-            else e = launch_wide<64>(c->kv_dtype, p, n_wg, s);
+            else e = launch_wide<64>(c->kv_dtype, p, n_wg + n_more, s);
         }
     }
     if (e == hipSuccess && (stages & kRead)) {

@@ -60,7 +60,7 @@ __device__ __forceinline__ void upper_many(const uint32_t *arr, uint32_t n, cons
 
 // One 1024-thread workgroup packs the batch.  `verdict` (may be null): a copy of the status this
 // workgroup writes, for callers that read it from elsewhere (the attention workspace header).
-__device__ void pack_rows_block(uint32_t n_seqs, const uint32_t *seq_slots, const uint32_t *q_lens,
+__device__ __forceinline__ void pack_rows_block(uint32_t n_seqs, const uint32_t *seq_slots, const uint32_t *q_lens,
                                 const uint32_t *cached, const uint32_t *pages, uint32_t stride,
                                 uint32_t page_shift, uint32_t pool_pages, uint32_t context,
                                 uint32_t max_rows, uint32_t *cu, uint32_t *positions,
@@ -255,7 +255,7 @@ constexpr uint32_t kCheckThreads = 256, kCheckGroups = 64;
 // of the entries (bit 0: a page outside the pool, bit 1: a missing cached page), uniform over
 // the workgroup.
 template <uint32_t T>
-__device__ uint32_t table_check_scan(uint32_t grp, uint32_t ngrp, uint32_t n_seqs,
+__device__ __forceinline__ uint32_t table_check_scan(uint32_t grp, uint32_t ngrp, uint32_t n_seqs,
                                      const uint32_t *seq_slots, const uint32_t *q_lens,
                                      const uint32_t *cached, const uint32_t *pages, uint32_t stride,
                                      uint32_t page_shift, uint32_t pool_pages, uint32_t context) {
@@ -320,7 +320,7 @@ __device__ __forceinline__ uint32_t table_failure(uint32_t bits) {
 // table_check_kernel's workgroup: the checks, and on a failure the batch rejected as the
 // packing rejects one and the status raised to it unless it holds a failure the reference
 // checks earlier.
-__device__ void table_check_block(uint32_t grp, uint32_t ngrp, uint32_t n_seqs,
+__device__ __forceinline__ void table_check_block(uint32_t grp, uint32_t ngrp, uint32_t n_seqs,
                                   const uint32_t *seq_slots, const uint32_t *q_lens,
                                   const uint32_t *cached, const uint32_t *pages, uint32_t stride,
                                   uint32_t page_shift, uint32_t pool_pages, uint32_t context,

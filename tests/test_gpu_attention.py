@@ -484,3 +484,45 @@ def test_ranges_of_small_batches(lia, wl, label, new, cached, hq, hkv, d, kv, ou
     print(f"[case] {label}: {units} units, {blocks} blocks, {ranges} ranges", flush=True)
     assert overflow == 0 and ranges <= max(8, blocks)
     assert (ranges == units) if one else (ranges > units or blocks == units)
+
+
+@pytest.mark.parametrize("kv,out,d", [(BF16, BF16, 64), (FP8, BF16, 128), (F16, F32, 64)])
+def test_prefill_queue(lia, wl, kv, out, d):
+    """More prefill units than workgroups, of many lengths, with two long rows among them: the plan
+    lists every unit as an item of its own (the long ones in pieces), longest first, past the
+    workgroups of one dispatch.  Outputs against the float64 oracle, through the fused two-launch plan
+    of lia_pack_plan_device as well, bit for bit the same."""
+    rng = np.random.default_rng(71)
+    new = np.concatenate([rng.integers(17, 240, 68), [1, 1]])
+    cached = np.concatenate([rng.integers(0, 700, 68), [6000, 5111]])
+    g = wl.Geometry(hq=8, hkv=8, d=d, kv_dtype=kv, q_dtype=BF16, out_dtype=out)
+    b = wl.custom(new + cached, new, geom=g, seed=71)
+    case = G.Case(b, seed=71)
+    got, _ = _check(case, lia, f"prefill queue kv={kv} d={d}")
+    units, blocks, items, overflow = case.last_ws[:16].view(torch.int32).tolist()
+    print(f"[case] prefill queue: {units} units, {items} items", flush=True)
+    assert overflow == 0 and units > 512 and items > units
+    dev, cfg = case.device(), case.config(lia)
+    z = lambda n: torch.full((n,), -7, dtype=torch.int32, device="cuda")  # noqa: E731
+    cu, pos, seq, slots, status = z(b.n_seqs + 1), z(b.n_rows), z(b.n_rows), z(b.n_rows), z(1)
+    ws = G.dirty_workspace(lia, cfg)
+    o = torch.zeros((b.n_rows, g.hq, d), dtype=torch.float32 if out == F32 else torch.bfloat16, device="cuda")
+    lia.pack_plan_device(cfg, G.u32_dev(np.arange(b.n_seqs)), G.u32_dev(b.q_len), G.u32_dev(b.cached), dev["pages"],
+                         b.n_rows, b.stride * g.page_size, cu, pos, seq, slots, status, ws)
+    lia.attention_partial(cfg, b.n_seqs, dev["pages"], dev["q"], dev["kc"], dev["vc"], o, ws, dev["k_scales"],
+                          dev["v_scales"])
+    lia.attention_merge(cfg, b.n_seqs, b.n_rows, o, ws)
+    torch.cuda.synchronize()
+    assert status.item() == 0 and ws[:16].view(torch.int32).tolist() == [units, blocks, items, 0]
+    assert np.array_equal(o.float().cpu().numpy(), got)
+    # a rejected step (a page outside the pool) leaves the output alone: no item of the queue runs
+    bad = b.flat_table()
+    bad[b.stride * 3] = b.pool_pages + 1
+    o.fill_(7.0)
+    lia.pack_plan_device(cfg, G.u32_dev(np.arange(b.n_seqs)), G.u32_dev(b.q_len), G.u32_dev(b.cached), G.u32_dev(bad),
+                         b.n_rows, b.stride * g.page_size, cu, pos, seq, slots, status, ws)
+    lia.attention_partial(cfg, b.n_seqs, dev["pages"], dev["q"], dev["kc"], dev["vc"], o, ws, dev["k_scales"],
+                          dev["v_scales"])
+    lia.attention_merge(cfg, b.n_seqs, b.n_rows, o, ws)
+    torch.cuda.synchronize()
+    assert status.item() != 0 and torch.all(o == 7.0)
