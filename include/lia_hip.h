@@ -540,9 +540,12 @@ int lia_schedule_rows(lia_page_cache *cache, uint32_t n_slots, lia_request *requ
  *     (ties: larger id) and (max, f64 mass) normalizers.  Device pointers, async on stream.
  *   lia_sample_host: the host tail on host copies of those records (logits: the full rows,
  *     read only for a nucleus fallback).
- *   lia_sample_paged: the whole tail: temperatures up, kernel, records down, per-row
- *     sampling, full-row reads for fallbacks; synchronises the stream (as the reference).
- *     workspace (device) and host buffers of lia_nucleus_workspace_bytes / _host_bytes.
+ *   lia_sample_paged: the whole tail: temperatures up, kernels, row summaries down (the 128
+ *     best candidates, maximum, mass and bound), per-row sampling, the records of rows that a
+ *     summary does not settle, full-row reads for fallbacks; synchronises the stream (as the
+ *     reference).  workspace (device) and host buffers of lia_nucleus_workspace_bytes /
+ *     _host_bytes; a workspace without the summaries' room (1,056 bytes a row, from 13 parts of the
+ *     vocabulary) is taken too, and every row's records are read.
  * samplers[i] == NULL selects greedy for output row i; positions[i] is the row's position
  * (Sampling::set_position).  *fallbacks counts full-row reads (nucleus_fallbacks).
  */
