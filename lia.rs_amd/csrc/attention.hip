@@ -2375,7 +2375,10 @@ __global__ __launch_bounds__(WCfg<D>::THREADS, 2) void wide_kernel(AttnParams p)
     asm volatile("" ::"s"(wd.unit), "s"(wd.lo), "s"(wd.hi), "s"(wd.flags), "s"(wd.first.block_start),
                  "s"(wd.first.nblocks), "s"(wd.first.cblocks), "s"(wd.first.rowbeg), "s"(wd.first.nrows_hk),
                  "s"(wd.first.kend), "s"(wd.first.table_row), "s"(wd.first.kcache));
-    if (wg >= p.n_wg && wg >= p.header[2]) return; // past the queue (or the plan has none)
+    if (wg >= p.n_wg && wg >= p.header[2]) { // past the queue (or the plan has none)
+        if (p.newk) append_rows<D, KVT>(p, wg, gridDim.x);
+        return;
+    }
     const uint32_t tid = threadIdx.x, lane = tid & 63;
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
     const uint32_t g = lane >> 4, li = lane & 15;

@@ -90,6 +90,21 @@ def test_fused_prefill_chunks(lia, wl, hq, hkv):
     _check(G.Case(wl.custom(ctx, q, geom=g, seed=15), seed=15), lia, f"prefill hq={hq} hkv={hkv}", 15)
 
 
+@pytest.mark.parametrize("kv,d", [(BF16, 128), (F16, 64)])
+def test_fused_prefill_queue(lia, wl, kv, d):
+    """A queued prefill (more units than workgroups of one dispatch): every new row reaches the pool,
+    whatever the number of workgroups launched past the queue's end."""
+    rng = np.random.default_rng(19)
+    new = np.concatenate([rng.integers(17, 240, 68), [1, 1]])
+    cached = np.concatenate([rng.integers(0, 500, 68), [6000, 5111]])
+    g = wl.Geometry(hq=8, hkv=8, d=d, kv_dtype=kv)
+    case = G.Case(wl.custom(new + cached, new, geom=g, seed=19), seed=19)
+    case.run(lia)
+    units, _, items, overflow = case.last_ws[:16].view(torch.int32).tolist()
+    assert overflow == 0 and units > 512 and items > units
+    _check(case, lia, f"prefill queue kv={kv} d={d}", 19)
+
+
 @pytest.mark.parametrize("q_len", [[1, 0, 3, 0, 1], [0, 2, 0, 64, 0]])
 def test_fused_sequences_without_rows(lia, wl, q_len):
     """Sequences adding no rows next to decode, MTP and prefill rows, through the fused launch."""
