@@ -116,6 +116,20 @@ int lia_pack_rows(const lia_paging_limits *limits, const lia_paged_row *rows, ui
                   uint32_t *sequences, uint32_t *flat_pages, lia_group *groups,
                   uint32_t *cu_seqlens, uint32_t *slot_mapping, lia_pack_info *info);
 
+/*
+ * Whether a packed step's rows may be appended by the attention launch that reads the pool
+ * (lia_attention_partial_append): 1 when no cached key of any group (a position below its first
+ * row's) lies in a slot the step writes, else 0.  lia_pack_rows accepts steps of the second kind: a
+ * sequence whose rows lie in several groups, a page that one sequence attends and another writes.
+ * Their rows are appended by a launch of their own (lia_kv_append) before the attention.  The arrays
+ * are lia_pack_rows' outputs.  No counterpart in the reference, whose append is always its own launch
+ * (src/inference/llama.rs:253-288).
+ */
+int lia_append_fusable(const lia_paging_limits *limits, uint32_t n_rows, uint32_t n_groups,
+                       const uint32_t *positions, const uint32_t *sequences,
+                       const uint32_t *flat_pages, const uint32_t *cu_seqlens,
+                       const uint32_t *slot_mapping);
+
 /* decode_span / decode_parts (src/inference/llama.rs:15-35) without the env override. */
 uint32_t lia_decode_span(uint32_t tokens);
 uint32_t lia_decode_parts(uint32_t tokens, uint32_t span);
@@ -356,9 +370,10 @@ int lia_attention_merge(const lia_attention_config *config, uint32_t n_seqs, uin
  * aligned.  The plan must come from the same packed rows: the first row of each sequence
  * sits at the sequence's cached length and its rows' keys are read from new_k / new_v, the
  * cached keys from the pool.  The pool afterwards holds the same bytes lia_kv_append
- * writes.  No cached key of any sequence may live in a slot this step writes (the
- * reference's page ownership guarantees it: packing rejects duplicate slots and new rows
- * go to the sequence's own pages).
+ * writes.  No cached key of any sequence may live in a slot this step writes: the launch reads
+ * such a key before or after it is written, as it comes.  The page cache's tables never bring it
+ * about (a page is written by one sequence, and attended by others once it is full); packing alone
+ * does not exclude it, lia_append_fusable says whether a packed step is free of it.
  */
 int lia_attention_partial_append(const lia_attention_config *config, uint32_t n_seqs,
                                  uint32_t n_rows, const uint32_t *pages,

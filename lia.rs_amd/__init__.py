@@ -119,6 +119,8 @@ EXPORTS = {
                                 C.c_void_p, C.c_void_p, C.c_uint32, C.c_void_p, C.c_uint32,
                                 C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p,
                                 C.c_void_p, C.POINTER(PackInfo)]),
+    "lia_append_fusable": (C.c_int, [C.POINTER(PagingLimits), C.c_uint32, C.c_uint32, C.c_void_p,
+                                     C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p]),
     "lia_decode_span": (C.c_uint32, [C.c_uint32]),
     "lia_decode_parts": (C.c_uint32, [C.c_uint32, C.c_uint32]),
     "lia_pack_device": (C.c_int, [C.c_uint32, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p,
@@ -913,11 +915,13 @@ class Engine:
         image = self._meta_host.numpy()
         spans = {k: slice(int(b), int(b) + n) for (k, n), b in zip(sizes.items(), starts)}
         self._meta_image = {k: image[x] for k, x in spans.items()}
+        at = {k: v.ctypes.data for k, v in self._meta_image.items()}
+        self._fusable_args = [at[k] for k in ("positions", "sequences", "pages", "cu_seqlens", "slot_mapping")]
         self.paging = dict(
             stride=stride,
             **{k: self._meta[x] for k, x in spans.items()},
             workspace=torch.zeros(workspace_bytes(self.config), dtype=torch.uint8, device=dev),
-            n_seqs=0, n_rows=0, refused=None)
+            n_seqs=0, n_rows=0, refused=None, fusable=False)
         torch.cuda.synchronize()
 
     def stage(self, rows, tables, outputs=()):
@@ -937,6 +941,7 @@ class Engine:
             image[key][:len(value)] = value.view(np.int32)
         self._meta.copy_(self._meta_host, non_blocking=True)
         w["n_seqs"], w["n_rows"] = ng, n
+        w["fusable"] = lib().lia_append_fusable(C.byref(self.limits), n, ng, *self._fusable_args) == 1
         # the step's work list, the same for every layer; a geometry the kernels refuse is attention()'s
         # to report
         w["refused"] = None
@@ -951,8 +956,9 @@ class Engine:
     def attention(self, layer, q, k, v, out=None):
         """Append this step's K/V rows to layer's pool and attend (llama.rs:203-288), on the plan
         stage() made.  Rows of the pool's type (bf16 on an FP8 pool) are appended by the attention
-        call itself, others by a launch before it: two or three launches a layer where append,
-        plan, attention and combine were four."""
+        call itself, on a 16-bit pool where no staged sequence attends a slot the step writes; others
+        by a launch before it: two or three launches a layer where append, plan, attention and
+        combine were four."""
         import torch
         w = self.paging
         n = w["n_rows"]
@@ -967,7 +973,8 @@ class Engine:
         ks, vs = self.k_scales[layer], self.v_scales[layer]
         fp8 = self.kv_dtype == FP8
         args = self.config, w["n_seqs"], w["pages"]
-        fused = (k.dtype == v.dtype and torch_dtype_code(k.dtype) == (BF16 if fp8 else self.kv_dtype)
+        fused = ((fp8 or w["fusable"]) and k.dtype == v.dtype
+                 and torch_dtype_code(k.dtype) == (BF16 if fp8 else self.kv_dtype)
                  and (k.data_ptr() | v.data_ptr()) % 16 == 0)
         if fused and fp8:
             attention_partial_append_fp8(*args, w["slot_mapping"], q, k, v, kc, vc, ks, vs, out,

@@ -5,6 +5,7 @@
 #include <stdint.h>
 #include <string.h>
 
+#include <new>
 #include <unordered_map>
 #include <unordered_set>
 #include <vector>
@@ -111,4 +112,32 @@ extern "C" int lia_pack_rows(const lia_paging_limits *lim, const lia_paged_row *
     info->parts = decoding ? lia_decode_parts(maximum, span) : (maximum + span - 1) / span;
     info->n_groups = n_groups;
     return LIA_OK;
+}
+
+extern "C" int lia_append_fusable(const lia_paging_limits *lim, uint32_t n_rows, uint32_t n_groups,
+                                  const uint32_t *positions, const uint32_t *sequences,
+                                  const uint32_t *flat_pages, const uint32_t *cu_seqlens,
+                                  const uint32_t *slot_mapping) {
+    if (!lim || lim->page_size == 0 || !positions || !sequences || !flat_pages || !cu_seqlens || !slot_mapping)
+        return LIA_E_ARG;
+    const uint32_t P = lim->page_size, stride = (lim->context + P - 1) / P;
+    try {
+        std::vector<bool> written(lim->pool_pages); // pages the step writes into
+        for (uint32_t r = 0; r < n_rows; r++)
+            if (slot_mapping[r] / P < lim->pool_pages) written[slot_mapping[r] / P] = true;
+        for (uint32_t g = 0; g < n_groups; g++) {
+            const uint32_t first = cu_seqlens[g], cached = positions[first];
+            const uint32_t *table = flat_pages + (size_t)sequences[first] * stride;
+            for (uint32_t e = 0; e * P < cached; e++) {
+                if (table[e] >= lim->pool_pages || !written[table[e]]) continue;
+                // few come here: a group's own last page, and pages that sequences share
+                const uint32_t keys = cached - e * P < P ? cached - e * P : P;
+                for (uint32_t r = 0; r < n_rows; r++)
+                    if (slot_mapping[r] / P == table[e] && slot_mapping[r] % P < keys) return 0;
+            }
+        }
+    } catch (const std::bad_alloc &) {
+        return 0; // appending first is right for every batch
+    }
+    return 1;
 }

@@ -355,6 +355,49 @@ def test_engine_attention_appends_and_attends(lia, O, kv, src, offset):
             assert err.max() < (5e-2 if kv == FP8 else 2e-2) and err.mean() < (5e-3 if kv == FP8 else 2e-3)
 
 
+@pytest.mark.parametrize("kv", [F16, BF16])
+@pytest.mark.parametrize("case", ["interleaved", "shared", "interleaved prefill", "shared prefill"])
+def test_engine_attends_rows_the_step_appends(lia, O, kv, case):
+    """Steps in which a cached key of one group is a row that the same step appends, with rows of the
+    pool's type: one sequence in two groups, and a page that one sequence writes and another attends, as
+    decode and as prefill batches.  The rows' slots hold garbage before; outputs against the float64
+    oracle over the pool after the append."""
+    eng = lia.Engine(16, 2, 128, pool_tokens=2048, layers=1, page_size=32, kv_dtype=kv, prefill_batch=256)
+    eng.configure_paging(4, 1024)
+    rng = np.random.default_rng(23)
+    free = [int(p) for p in rng.permutation(64)]
+    tables = [free[:8], free[8:28]]
+    span = lambda s, a, b: [(1, p, s) for p in range(a, b)]  # noqa: E731
+    if case == "interleaved":
+        rows = span(0, 100, 101) + span(1, 500, 501) + span(0, 101, 102)
+    elif case == "interleaved prefill":
+        rows = span(0, 100, 140) + span(1, 500, 535) + span(0, 140, 200)
+    else:  # sequence 1 attends page 3 of sequence 0 in its own place 1
+        tables[1][1] = tables[0][3]
+        rows = (span(0, 127, 128) + span(1, 500, 501) if case == "shared"
+                else span(0, 90, 150) + span(1, 500, 540))
+    packed = eng.stage(rows, tables, outputs=[0])
+    n = len(rows)
+    pool = [O.from_f32(rng.standard_normal((2048, 2, 128)).astype(np.float32), kv) for _ in "kv"]
+    for a in pool:
+        a[packed["slot_mapping"]] = O.from_f32(np.full((n, 2, 128), 50.0, np.float32), kv)
+    for dst, a in zip((eng.k[0], eng.v[0]), pool):
+        dst.view(torch.int16).copy_(G.to_dev(a.view(np.int16)))
+    tdt = torch.float16 if kv == F16 else torch.bfloat16
+    q = rng.standard_normal((n, 16, 128)).astype(np.float32)
+    new = [O.from_f32(rng.standard_normal((n, 2, 128)).astype(np.float32), kv) for _ in "kv"]
+    out = eng.attention(0, G.to_dev(q), *[G.to_dev(a, tdt) for a in new])
+    torch.cuda.synchronize()
+    for a, x in zip(pool, new):
+        a[packed["slot_mapping"]] = x
+    assert np.array_equal(eng.k[0].cpu().numpy().view(np.uint16), pool[0])
+    assert np.array_equal(eng.v[0].cpu().numpy().view(np.uint16), pool[1])
+    ref = O.attention_f64(O.geom(16, 2, 128, 32, packed["stride"], kv), packed["positions"], packed["sequences"],
+                          packed["flat"], q, pool[0].reshape(-1), pool[1].reshape(-1))
+    err = np.abs(out.cpu().numpy() - ref)
+    assert err.max() < 2e-2 and err.mean() < 2e-3
+
+
 def _pack_both(lia, q_len, cached, tables, P, pool):
     """The device's packing (both entry points' checks) and the host's, of one batch: their metadata,
     or their failure codes."""
