@@ -922,11 +922,14 @@ class Engine:
             **{k: self._meta[x] for k, x in spans.items()},
             workspace=torch.zeros(workspace_bytes(self.config), dtype=torch.uint8, device=dev),
             n_seqs=0, n_rows=0, refused=None, fusable=False)
+        # The staged step's plan and records lie apart from paging["workspace"], which is the caller's
+        # for calls of its own: one made between two layers leaves the plan alone.
+        self._step_workspace = torch.empty_like(self.paging["workspace"])
         torch.cuda.synchronize()
 
     def stage(self, rows, tables, outputs=()):
         """Host packing + metadata upload of Engine::run_paged (paging.rs:118-237), and the plan
-        attention() works from: the engine's workspace is the step's until its last layer."""
+        attention() works from, in the engine's own workspace."""
         import torch
         if self.paging is None:
             raise LiaError(-19, "paging is not configured")
@@ -947,7 +950,7 @@ class Engine:
         w["refused"] = None
         try:
             attention_plan(self.config, ng, n, w["cu_seqlens"], w["positions"], w["sequences"],
-                           w["workspace"], w["pages"])
+                           self._step_workspace, w["pages"])
         except LiaError as e:
             w["refused"] = e
         torch.cuda.current_stream().synchronize()
@@ -972,20 +975,19 @@ class Engine:
         k, v, kc, vc = k.reshape(n, -1), v.reshape(n, -1), self.k[layer], self.v[layer]
         ks, vs = self.k_scales[layer], self.v_scales[layer]
         fp8 = self.kv_dtype == FP8
-        args = self.config, w["n_seqs"], w["pages"]
+        args, ws = (self.config, w["n_seqs"], w["pages"]), self._step_workspace
         fused = ((fp8 or w["fusable"]) and k.dtype == v.dtype
                  and torch_dtype_code(k.dtype) == (BF16 if fp8 else self.kv_dtype)
                  and (k.data_ptr() | v.data_ptr()) % 16 == 0)
         if fused and fp8:
-            attention_partial_append_fp8(*args, w["slot_mapping"], q, k, v, kc, vc, ks, vs, out,
-                                         w["workspace"])
+            attention_partial_append_fp8(*args, w["slot_mapping"], q, k, v, kc, vc, ks, vs, out, ws)
         elif fused:
-            attention_partial_append(*args, w["slot_mapping"], q, k, v, kc, vc, out, w["workspace"])
+            attention_partial_append(*args, w["slot_mapping"], q, k, v, kc, vc, out, ws)
         else:
             layout = KVLayout(self.hkv, self.d, self.page_size, self.pool_pages, self.kv_dtype)
             kv_append(layout, k, v, kc, vc, slot_mapping=w["slot_mapping"], k_scales=ks, v_scales=vs)
-            attention_partial(*args, q, kc, vc, out, w["workspace"], ks, vs)
-        attention_merge(self.config, w["n_seqs"], n, out, w["workspace"])
+            attention_partial(*args, q, kc, vc, out, ws, ks, vs)
+        attention_merge(self.config, w["n_seqs"], n, out, ws)
         return out
 
     def _transfer(self):

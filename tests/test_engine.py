@@ -13,10 +13,14 @@ LAUNCHES = ("attention_plan", "kv_append", "attention_partial", "attention_parti
 
 @pytest.fixture
 def engine(lia, monkeypatch):
-    """engine(kv_dtype) -> an Engine on host memory; its `calls` lists the launches by name."""
-    calls = []
+    """engine(kv_dtype) -> an Engine on host memory that records its launches."""
+    calls, used = [], set()
     for name in LAUNCHES:
-        monkeypatch.setattr(lia, name, lambda *a, _name=name, **k: calls.append(_name))
+        def record(*a, _name=name, **k):
+            calls.append(_name)
+            used.update(t.data_ptr() for t in a if isinstance(t, torch.Tensor))
+
+        monkeypatch.setattr(lia, name, record)
     stream = types.SimpleNamespace(cuda_stream=0, synchronize=lambda: calls.append("synchronize"))
     monkeypatch.setattr(torch.cuda, "current_stream", lambda *a: stream)
     monkeypatch.setattr(torch.cuda, "synchronize", lambda *a: None)
@@ -27,7 +31,7 @@ def engine(lia, monkeypatch):
         e = lia.Engine(16, 2, 128, pool_tokens=2048, layers=1, page_size=32, kv_dtype=kv_dtype,
                        prefill_batch=64, device="cpu")
         e.configure_paging(maximum_sequences, 1024)
-        e.calls = calls
+        e.calls, e.used = calls, used  # names of the launches, addresses of their tensors
         return e
 
     return make
@@ -82,3 +86,12 @@ def test_append_fusable_equals_a_search_of_every_cached_key(lia):
         assert fusable == (not read & set(got["slot_mapping"].tolist()))
         seen.add(fusable)
     assert seen == {0, 1}
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+def test_a_staged_plan_lies_apart_from_the_callers_workspace(engine, dtype):
+    """paging["workspace"] may serve other calls between stage() and the last layer."""
+    e = engine()
+    e.stage(*PRIVATE)
+    attend(e, 3, dtype)
+    assert e._step_workspace.data_ptr() in e.used and e.paging["workspace"].data_ptr() not in e.used

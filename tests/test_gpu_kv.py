@@ -398,6 +398,25 @@ def test_engine_attends_rows_the_step_appends(lia, O, kv, case):
     assert err.max() < 2e-2 and err.mean() < 2e-3
 
 
+def test_engine_layers_around_other_calls(lia):
+    """A layer's output does not change when, after stage(), another batch runs on paging["workspace"]."""
+    eng = lia.Engine(16, 2, 128, pool_tokens=4096, layers=1, page_size=32, prefill_batch=64)
+    eng.configure_paging(4, 2048)
+    g = torch.Generator(device="cuda").manual_seed(5)
+    rand = lambda *s: torch.randn(s, generator=g, device="cuda")  # noqa: E731
+    for x in (eng.k[0], eng.v[0]):
+        x.view(torch.float16).copy_(rand(4096, 2, 128))
+    tables = [list(range(60)), list(range(60, 124))]
+    rows = [(1, 1500, 0), (1, 2000, 1)]
+    q, k, v = rand(2, 16, 128), rand(2, 2, 128).half(), rand(2, 2, 128).half()
+    eng.stage(rows, tables, [0, 1])
+    want = eng.attention(0, q, k, v).clone()
+    w = eng.paging
+    lia.paged_attention(eng.config, 1, w["cu_seqlens"], w["positions"], w["sequences"], w["pages"], q[:1],
+                        eng.k[0], eng.v[0], torch.empty((1, 16, 128), device="cuda"), w["workspace"])
+    assert torch.equal(eng.attention(0, q, k, v), want)
+
+
 def _pack_both(lia, q_len, cached, tables, P, pool):
     """The device's packing (both entry points' checks) and the host's, of one batch: their metadata,
     or their failure codes."""
