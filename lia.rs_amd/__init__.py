@@ -961,7 +961,7 @@ class Engine:
         stage() made.  Rows of the pool's type (bf16 on an FP8 pool) are appended by the attention
         call itself, on a 16-bit pool where no staged sequence attends a slot the step writes; others
         by a launch before it: two or three launches a layer where append, plan, attention and
-        combine were four."""
+        combine were four, as they still are in a captured graph."""
         import torch
         w = self.paging
         n = w["n_rows"]
@@ -975,6 +975,14 @@ class Engine:
         k, v, kc, vc = k.reshape(n, -1), v.reshape(n, -1), self.k[layer], self.v[layer]
         ks, vs = self.k_scales[layer], self.v_scales[layer]
         fp8 = self.kv_dtype == FP8
+        if torch.cuda.is_current_stream_capturing():
+            # a replay serves whatever is staged then: the graph holds the rows' append, which no step
+            # forbids, and a plan of the metadata it finds
+            layout = KVLayout(self.hkv, self.d, self.page_size, self.pool_pages, self.kv_dtype)
+            kv_append(layout, k, v, kc, vc, slot_mapping=w["slot_mapping"], k_scales=ks, v_scales=vs)
+            paged_attention(self.config, w["n_seqs"], w["cu_seqlens"], w["positions"], w["sequences"],
+                            w["pages"], q, kc, vc, out, w["workspace"], ks, vs)
+            return out
         args, ws = (self.config, w["n_seqs"], w["pages"]), self._step_workspace
         fused = ((fp8 or w["fusable"]) and k.dtype == v.dtype
                  and torch_dtype_code(k.dtype) == (BF16 if fp8 else self.kv_dtype)

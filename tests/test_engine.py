@@ -24,6 +24,7 @@ def engine(lia, monkeypatch):
     stream = types.SimpleNamespace(cuda_stream=0, synchronize=lambda: calls.append("synchronize"))
     monkeypatch.setattr(torch.cuda, "current_stream", lambda *a: stream)
     monkeypatch.setattr(torch.cuda, "synchronize", lambda *a: None)
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
     zeros = torch.zeros
     monkeypatch.setattr(torch, "zeros", lambda *a, pin_memory=False, **k: zeros(*a, **k))
 
@@ -95,3 +96,11 @@ def test_a_staged_plan_lies_apart_from_the_callers_workspace(engine, dtype):
     e.stage(*PRIVATE)
     attend(e, 3, dtype)
     assert e._step_workspace.data_ptr() in e.used and e.paging["workspace"].data_ptr() not in e.used
+
+
+def test_a_captured_layer_plans_and_appends_for_itself(engine, monkeypatch):
+    """The graph of a layer is replayed for later steps, which may attend rows that they append."""
+    e = engine()
+    e.stage(*PRIVATE)
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: True)
+    assert attend(e, 3, torch.float16) == ["kv_append", "paged_attention"]

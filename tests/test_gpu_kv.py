@@ -417,6 +417,45 @@ def test_engine_layers_around_other_calls(lia):
     assert torch.equal(eng.attention(0, q, k, v), want)
 
 
+def test_engine_layer_replayed_for_later_steps(lia):
+    """A captured layer, replayed after other steps of its shape were staged (private pages, a page that
+    the step writes and attends, private pages of other contexts), equals the eager layer of each step,
+    whose later layers the replay leaves alone."""
+    eng = lia.Engine(16, 2, 128, pool_tokens=4096, layers=1, page_size=32, prefill_batch=64)
+    eng.configure_paging(4, 2048)
+    g = torch.Generator(device="cuda").manual_seed(7)
+    rand = lambda *s: torch.randn(s, generator=g, device="cuda")  # noqa: E731
+    pool = [rand(4096, 2, 128).half() for _ in "kv"]
+    q, k, v = rand(2, 16, 128), rand(2, 2, 128).half(), rand(2, 2, 128).half()
+    out = torch.empty((2, 16, 128), device="cuda")
+
+    def refill():
+        for dst, src in zip((eng.k[0], eng.v[0]), pool):
+            dst.view(torch.float16).copy_(src)
+
+    private, shared = [list(range(60)), list(range(60, 124))], [list(range(60)), [*range(60, 70), 46, *range(70, 120)]]
+    eng.stage([(1, 1500, 0), (1, 1900, 1)], private, [0, 1])
+    eng.attention(0, q, k, v, out)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        eng.attention(0, q, k, v, out)
+    for tables, at in ((private, (1500, 1900)), (shared, (1500, 1900)), (private, (70, 333)), (shared, (1501, 700))):
+        eng.stage([(1, at[0], 0), (1, at[1], 1)], tables, [0, 1])
+        refill()
+        want = eng.attention(0, q, k, v).clone()
+        pools = eng.k[0].clone(), eng.v[0].clone()
+        refill()
+        out.fill_(float("nan"))
+        graph.replay()
+        torch.cuda.synchronize()
+        # the eager layer may read the new rows apart from the cached ones: f16 weights of other chunks,
+        # each rounded by at most 2^-11
+        assert (out - want).abs().max() <= 2e-3 * want.abs().max()
+        assert torch.equal(eng.k[0], pools[0]) and torch.equal(eng.v[0], pools[1])
+        refill()
+        assert torch.equal(eng.attention(0, q, k, v), want)
+
+
 def _pack_both(lia, q_len, cached, tables, P, pool):
     """The device's packing (both entry points' checks) and the host's, of one batch: their metadata,
     or their failure codes."""
