@@ -942,18 +942,19 @@ class Engine:
                            ("slot_mapping", packed["slot_mapping"]), ("pages", packed["flat"]),
                            ("cu_seqlens", packed["cu_seqlens"])):
             image[key][:len(value)] = value.view(np.int32)
-        self._meta.copy_(self._meta_host, non_blocking=True)
         w["n_seqs"], w["n_rows"] = ng, n
         w["fusable"] = lib().lia_append_fusable(C.byref(self.limits), n, ng, *self._fusable_args) == 1
         # the step's work list, the same for every layer; a geometry the kernels refuse is attention()'s
         # to report
         w["refused"] = None
-        try:
-            attention_plan(self.config, ng, n, w["cu_seqlens"], w["positions"], w["sequences"],
-                           self._step_workspace, w["pages"])
-        except LiaError as e:
-            w["refused"] = e
-        torch.cuda.current_stream().synchronize()
+        with torch.cuda.device(self._meta.device):  # the pool's, whichever is the caller's current one
+            self._meta.copy_(self._meta_host, non_blocking=True)
+            try:
+                attention_plan(self.config, ng, n, w["cu_seqlens"], w["positions"], w["sequences"],
+                               self._step_workspace, w["pages"])
+            except LiaError as e:
+                w["refused"] = e
+            torch.cuda.current_stream().synchronize()
         return packed
 
     def attention(self, layer, q, k, v, out=None):

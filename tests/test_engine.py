@@ -1,5 +1,6 @@
 """CPU tests of Engine's staging and launches: which calls a staged step makes, with the launches
 recorded instead of issued."""
+import contextlib
 import types
 
 import numpy as np
@@ -25,6 +26,14 @@ def engine(lia, monkeypatch):
     monkeypatch.setattr(torch.cuda, "current_stream", lambda *a: stream)
     monkeypatch.setattr(torch.cuda, "synchronize", lambda *a: None)
     monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+
+    @contextlib.contextmanager
+    def device(d):
+        calls.append(f"device {d}")
+        yield
+        calls.append("device back")
+
+    monkeypatch.setattr(torch.cuda, "device", device)
     zeros = torch.zeros
     monkeypatch.setattr(torch, "zeros", lambda *a, pin_memory=False, **k: zeros(*a, **k))
 
@@ -104,3 +113,10 @@ def test_a_captured_layer_plans_and_appends_for_itself(engine, monkeypatch):
     e.stage(*PRIVATE)
     monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: True)
     assert attend(e, 3, torch.float16) == ["kv_append", "paged_attention"]
+
+
+def test_stage_works_on_the_pools_device(engine):
+    """stage() only copied before; its plan is launched where the pool lies, not on the current device."""
+    e = engine()
+    e.stage(*PRIVATE)
+    assert e.calls == ["device cpu", "attention_plan", "synchronize", "device back"]
