@@ -954,7 +954,8 @@ class Engine:
                                self._step_workspace, w["pages"])
             except LiaError as e:
                 w["refused"] = e
-            torch.cuda.current_stream().synchronize()
+            finally:  # whatever was raised, the image is free when stage() ends
+                torch.cuda.current_stream().synchronize()
         return packed
 
     def attention(self, layer, q, k, v, out=None):

@@ -120,3 +120,16 @@ def test_stage_works_on_the_pools_device(engine):
     e = engine()
     e.stage(*PRIVATE)
     assert e.calls == ["device cpu", "attention_plan", "synchronize", "device back"]
+
+
+def test_an_interrupted_stage_ends_its_copy(engine, lia, monkeypatch):
+    """The next stage() writes the pinned image that the copy reads."""
+    e = engine()
+
+    def interrupted(*a):
+        raise KeyboardInterrupt
+
+    monkeypatch.setattr(lia, "attention_plan", interrupted)
+    with pytest.raises(KeyboardInterrupt):
+        e.stage(*PRIVATE)
+    assert "synchronize" in e.calls
