@@ -293,7 +293,7 @@ def pack_rows(limits, rows, tables, outputs=()):
     n = len(rows)
     try:
         row_arr = np.array(rows) if n else np.zeros((1, 3), np.uint32)
-    except ValueError:  # rows of different lengths
+    except (ValueError, TypeError):  # rows of different lengths, numbers numpy does not take
         row_arr = np.zeros(0)
     if row_arr.ndim == 2 and row_arr.shape[1] == 3 and row_arr.dtype.kind in "iu":
         row_arr = np.ascontiguousarray(row_arr.astype(np.uint32))

@@ -144,3 +144,27 @@ def test_partial_append_validates_before_launch(lia):
     assert call(F16, None, fake) == -20
     assert call(F16, fake, None) == -20
     assert call(F16, odd, fake) == -21
+
+
+class _Index:
+    """A whole number that numpy refuses to convert (as it does scalars on a device)."""
+
+    def __init__(self, value):
+        self.value = value
+
+    def __index__(self):
+        return self.value
+
+    def __array__(self, *args, **kwargs):
+        raise TypeError("not an array")
+
+
+def test_pack_rows_takes_whole_numbers_of_any_kind(lia):
+    """Rows are packed alike whether numpy can make an array of them or not."""
+    lim = lia.PagingLimits(4, 256, 32, 32, 1000, 64)
+    plain = [(1, 5, 0), (2, 6, 0), (3, 40, 1)]
+    tables = [[4], [7, 2]]
+    want = lia.pack_rows(lim, plain, tables)
+    for rows in (np.array(plain), [tuple(np.int64(x) for x in r) for r in plain], [tuple(_Index(x) for x in r) for r in plain]):
+        got = lia.pack_rows(lim, rows, tables)
+        assert all(np.array_equal(got[k], want[k]) for k in want)
