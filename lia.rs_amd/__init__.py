@@ -275,6 +275,14 @@ def _stream(stream=None):
     return _raw_stream()
 
 
+def _forget_stream():
+    global _raw_stream
+    _raw_stream = None
+
+
+os.register_at_fork(after_in_child=_forget_stream)  # torch then refuses the child's launches
+
+
 def torch_dtype_code(dt):
     import torch
     return {torch.float32: F32, torch.float16: F16, torch.bfloat16: BF16,

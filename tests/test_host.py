@@ -168,3 +168,12 @@ def test_pack_rows_takes_whole_numbers_of_any_kind(lia):
     for rows in (np.array(plain), [tuple(np.int64(x) for x in r) for r in plain], [tuple(_Index(x) for x in r) for r in plain]):
         got = lia.pack_rows(lim, rows, tables)
         assert all(np.array_equal(got[k], want[k]) for k in want)
+
+
+def test_a_forked_child_asks_torch_for_its_stream(lia, monkeypatch):
+    """The runtime does not survive a fork: torch says so to a child that asks it for a stream."""
+    monkeypatch.setattr(lia, "_raw_stream", lambda: 0)
+    child = os.fork()
+    if child == 0:
+        os._exit(0 if lia._raw_stream is None else 1)
+    assert os.waitstatus_to_exitcode(os.waitpid(child, 0)[1]) == 0
