@@ -111,12 +111,14 @@ __global__ __launch_bounds__(256) void nucleus_candidates_kernel(
     double sum = 0.0;
     const double t = temperatures[row];
     if (t > 0.0 && isfinite(mx)) {
-        // Quotients by the row's temperature from its reciprocal, corrected by a fused remainder:
-        // five operations, where the division sequence takes eleven.  Both sides are scaled to a
+        // Quotients by the row's temperature from its reciprocal, corrected by a fused remainder
+        // (Markstein, "Computation of elementary functions on the IBM RISC System/6000", 1990): five
+        // operations, where the division sequence takes eleven.  Both sides are scaled to a
         // temperature in [0.5, 1), and quotients below -1e6 (whose exponential is 0) cut, so no
-        // step leaves the exponent range.
+        // step leaves the exponent range.  An infinite temperature gives the weights of the largest
+        // finite one, 1 each.
         int e2;
-        const double ts = __builtin_frexp(t, &e2), inv = 1.0 / ts;
+        const double ts = __builtin_frexp(fmin(t, 0x1.fffffffffffffp1023), &e2), inv = 1.0 / ts;
 #pragma unroll
         for (uint32_t j = 0; j < kPerLane; j++) {
             const double x = fmax(__builtin_ldexp((double)v[j] - (double)mx, -e2), -1e6);

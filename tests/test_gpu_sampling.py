@@ -59,6 +59,13 @@ def test_candidates_special_values_and_ragged_vocab(lia):
         _check_records(lia, x, [1.0, 0.5, 1.0, 2.0, 0.0], f"special vocab={vocab}")
 
 
+def test_candidates_extreme_temperatures(lia):
+    rng = np.random.default_rng(10)
+    x = (rng.standard_normal((7, 1500)) * 4).astype(np.float32)
+    temps = [math.inf, 1.7976931348623157e308, 1e-300, 5e-324, math.nan, -1.0, -math.inf]
+    _check_records(lia, x, temps, "extreme temperatures")
+
+
 def test_candidates_minicpm5_vocabulary(lia):
     rng = np.random.default_rng(8)
     x = (rng.standard_normal((2, 130560)) * 3).astype(np.float32)
