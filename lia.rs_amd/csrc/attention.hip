@@ -224,6 +224,7 @@ struct PlanRule {
     uint32_t small_cost, span_shift;
     uint32_t n_more;     // work descriptors past n_wg (0: no queue)
     uint32_t rec;        // prefill: a record's cost (16ths of an eighth of a block); decode: 0
+    uint32_t room;       // units the list holds (a prefill plan's work descriptors lie behind them)
 };
 
 struct RawSeqs {
@@ -309,7 +310,7 @@ __device__ __forceinline__ void plan_lds(uint32_t n_seqs, const uint32_t *cu, co
         }
         lds_barrier();
     }
-    bool overflow = carry_units > max_units;
+    bool overflow = carry_units > rule.room;
     if constexpr (RAW) overflow |= carry_rows != raw.n_rows || raw_bad;
     const uint32_t U = overflow ? 0 : carry_units, B = overflow ? 0 : carry_blocks;
     // Work is split in cost: each unit's blocks are preceded by unit_cost virtual blocks (the
@@ -669,7 +670,7 @@ __global__ __launch_bounds__(256) void plan_kernel(uint32_t n_seqs, const uint32
                                                    const uint32_t *sequences, const uint32_t *pages,
                                                    uint32_t stride, uint32_t page_shift, uint32_t rpc,
                                                    uint32_t hkv, uint32_t max_units,
-                                                   uint32_t n_wg, uint32_t xcd, UnitDesc *units,
+                                                   uint32_t room, uint32_t n_wg, uint32_t xcd, UnitDesc *units,
                                                    WorkDesc *work, MergeDesc *merge,
                                                    uint32_t *header) {
     __shared__ uint32_t s_units[256], s_blocks[256];
@@ -704,8 +705,8 @@ __global__ __launch_bounds__(256) void plan_kernel(uint32_t n_seqs, const uint32
         }
         uint32_t u = carry_units + s_units[t] - nu;
         uint32_t blk = carry_blocks + s_blocks[t] - nb;
-        if (nu && u + nu > max_units) overflow = 1;
-        if (nu && u + nu <= max_units) {
+        if (nu && u + nu > room) overflow = 1;
+        if (nu && u + nu <= room) {
             uint32_t ncb = nu / hkv;
             const uint32_t cblocks = (p0 + 31) / 32;
             // KV head outermost: consecutive units (and the block ranges over them) stream
@@ -3105,7 +3106,7 @@ static int run_stages(int stages, const lia_attention_config *c, uint32_t n_seqs
     // descriptors past n_wg.  A prefill plan's descriptors therefore lie at the end of the unit list,
     // which is sized for the decode kernel's narrower units (where a configuration leaves the room;
     // it alone decides the place, as every array's of the workspace).
-    uint32_t n_more = 0;
+    uint32_t n_more = 0, room = L.max_units;
     if (NT == kWideNT) {
         const size_t hkv = c->num_kv_heads, rounds = 2 * p.round_wg;
         const size_t bound = ((size_t)n_rows / rpc + n_seqs) * hkv;
@@ -3114,6 +3115,7 @@ static int run_stages(int stages, const lia_attention_config *c, uint32_t n_seqs
         const size_t at = end > most * sizeof(WorkDesc) ? (end - most * sizeof(WorkDesc)) & ~(sizeof(WorkDesc) - 1) : 0;
         if (most >= n_wg && most <= L.max_units && at >= L.units + (most - rounds + 1) * sizeof(UnitDesc)) {
             work = (WorkDesc *)(ws + at);
+            room = (uint32_t)((at - L.units) / sizeof(UnitDesc)) - 1; // (the list ends with a unit of no blocks)
             if (bound > n_wg && parallel && bound / hkv <= kQueueGroups) n_more = (uint32_t)(bound + rounds) - n_wg;
         }
     }
@@ -3133,7 +3135,7 @@ static int run_stages(int stages, const lia_attention_config *c, uint32_t n_seqs
         const bool rec32 = p.out_f32 || c->kv_dtype == LIA_FP8_E4M3;
         const PlanRule rule{wide ? kUnitCostWide : kUnitCostDecode, lia_device_cus(), lag, xcd,
                             wide ? 1u << 18 : 6 * n_wg, wide ? 0u : 1u, n_more,
-                            wide ? (rec32 ? 9u : 5u) : 0u};
+                            wide ? (rec32 ? 9u : 5u) : 0u, room};
         if (pk && parallel) {
             // the packing, the plan (from the packing's inputs) and the table checks in one
             // launch, then the step's verdict
@@ -3168,7 +3170,7 @@ static int run_stages(int stages, const lia_attention_config *c, uint32_t n_seqs
             else
             e = launch<plan_kernel>(dim3(1), dim3(256), 0, s, n_seqs, cu_seqlens, positions,
                                     sequences, pages, c->stride, p.page_shift, rpc, c->num_kv_heads,
-                                    L.max_units, n_wg, rule.xcd, units, work, merge, header);
+                                    L.max_units, room, n_wg, rule.xcd, units, work, merge, header);
         }
     }
     if (e == hipSuccess && (stages & kPartial)) {

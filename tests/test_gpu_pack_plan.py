@@ -146,6 +146,23 @@ def test_pack_plan_rows_over_capacity_and_row_count_mismatch(lia, wl):
         assert hdr[0] == 0 and hdr[2] == 0, (q, hdr)
 
 
+@pytest.mark.parametrize("n_seqs,n_rows,rows,planned", [(1, 4096, 8192, True), (1, 4096, 20000, False),
+                                                        (1030, 16480, 8192, True), (1030, 16480, 80000, False)])
+def test_prefill_plan_of_more_units_than_its_list_holds(lia, n_seqs, n_rows, rows, planned):
+    """Metadata of other rows than the configuration's: a prefill plan whose units would reach the work
+    descriptors behind their list is empty, as one past the end of the list is (both plans)."""
+    cfg = lia.AttentionConfig(16, 2, 128, 16, 64, 2048, lia.BF16, lia.BF16, lia.BF16, 0.1, n_seqs, n_rows, 32768)
+    ws = torch.full((lia.workspace_bytes(cfg),), 0xA5, dtype=torch.uint8, device="cuda")
+    cu = torch.full((n_seqs + 1,), rows, dtype=torch.int32, device="cuda")
+    cu[0] = 0
+    meta = [torch.zeros(rows, dtype=torch.int32, device="cuda") for _ in range(2)]
+    lia.attention_plan(cfg, n_seqs, n_rows, cu, *meta, ws)
+    torch.cuda.synchronize()
+    hdr = ws[:32].view(torch.int32).cpu().numpy()
+    units = rows // 16 * 2 if planned else 0
+    assert hdr[0] == units and bool(hdr[2]) == planned and bool(hdr[3]) == (not planned)
+
+
 @pytest.mark.parametrize("n", [1, 5, 64, 300])
 def test_pack_plan_head_dim_64_decode(lia, wl, n):
     """head_dim 64 decode launches more workgroups (1,536) than the plan has threads (1,024): the
