@@ -410,9 +410,9 @@ extern "C" int lia_rope_coefficients(uint32_t rows, uint32_t head_dim, float bas
     if (head_dim != 64 && head_dim != 128) return LIA_E_UNSUPPORTED;
     if (((uintptr_t)coefficients & 7) != 0) return LIA_E_ALIGN;
     if (rows == 0) return LIA_OK;
-    // More rows a thread once that leaves every CU two workgroups: one, two and four rows a thread
-    // measured 2.94, 2.81 and 3.48 us at 512 groups (2,048 rows of 128), 4.27, 3.48 and 3.65 at
-    // 1,024, 6.56, 5.12 and 4.56 at 2,048.
+    // Two rows a thread from 512 workgroups of one row each (256 of two, one per CU), four from 2,048
+    // (512 of four, two per CU): one, two and four rows a thread measured 2.94, 2.81 and 3.48 us at 512
+    // (2,048 rows of 128), 4.27, 3.48 and 3.65 at 1,024, 6.56, 5.12 and 4.56 at 2,048.
     const uint32_t step = 256 / (head_dim / 2);
     const uint32_t groups = (uint32_t)(((uint64_t)rows + step - 1) / step);
     const uint32_t per = groups >= 2048 ? 4 : groups >= 512 ? 2 : 1;

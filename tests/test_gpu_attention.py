@@ -526,3 +526,19 @@ def test_prefill_queue(lia, wl, kv, out, d):
     lia.attention_merge(cfg, b.n_seqs, b.n_rows, o, ws)
     torch.cuda.synchronize()
     assert status.item() != 0 and torch.all(o == 7.0)
+
+
+@pytest.mark.parametrize("hq,hkv,kv,out,d", [(24, 8, BF16, BF16, 64), (25, 5, FP8, BF16, 128), (42, 7, F16, F32, 64)])
+def test_prefill_queue_of_other_group_sizes(lia, wl, hq, hkv, kv, out, d):
+    """A queue whose column blocks hold 42, 25 or 21 rows (groups of 3, 5 and 6 query heads a KV head,
+    also of an odd number of KV heads): every item's place and length by the sums for a row count that is
+    no power of two.  Outputs against the float64 oracle."""
+    rng = np.random.default_rng(72)
+    new = np.concatenate([rng.integers(17, 240, 36), [1]])
+    cached = np.concatenate([rng.integers(0, 700, 36), [6000]])
+    g = wl.Geometry(hq=hq, hkv=hkv, d=d, kv_dtype=kv, q_dtype=BF16, out_dtype=out)
+    case = G.Case(wl.custom(new + cached, new, geom=g, seed=72), seed=72)
+    _check(case, lia, f"prefill queue {hq}/{hkv} heads kv={kv} d={d}")
+    units, blocks, items, overflow = case.last_ws[:16].view(torch.int32).tolist()
+    print(f"[case] prefill queue: {units} units, {items} items", flush=True)
+    assert overflow == 0 and units > 512 and items > units

@@ -512,3 +512,19 @@ def test_pack_device_rows_sharing_a_page(lia, big, other, want):
         q_len, cached, tables = [4500] + q_len, [0] + cached, [list(range(100, 100 + -(-4500 // P)))] + tables
     status, host = _pack_both(lia, q_len, cached, tables, P, pool)
     assert status == host == want
+
+
+def test_pack_device_with_the_page_table_at_its_fullest(lia):
+    """1,023 sequences of two rows that straddle a page each, and one of 14,353 rows: 2,944 runs, nearly
+    all that the packing's rule lets into its table of 4,096 pages.  As the host packs them, and with a
+    slot written twice."""
+    P, q_len = 16, [2] * 1023 + [14353]
+    cached = [15] * 1023 + [0]
+    need = [2] * 1023 + [-(-14353 // P)]
+    perm = np.random.default_rng(31).permutation(sum(need) + 3)
+    tables = np.split(perm[:sum(need)], np.cumsum(need)[:-1])
+    status, want = _pack_both(lia, q_len, cached, tables, P, len(perm))
+    assert status == (want or 0) == 0
+    tables[700][1] = tables[20][1]
+    status, want = _pack_both(lia, q_len, cached, tables, P, len(perm))
+    assert status == want == 11
