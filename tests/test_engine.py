@@ -116,7 +116,7 @@ def test_a_captured_layer_plans_and_appends_for_itself(engine, monkeypatch):
 
 
 def test_stage_works_on_the_pools_device(engine):
-    """stage() only copied before; its plan is launched where the pool lies, not on the current device."""
+    """The plan is launched where the pool lies, whichever device is current."""
     e = engine()
     e.stage(*PRIVATE)
     assert e.calls == ["device cpu", "attention_plan", "synchronize", "device back"]
